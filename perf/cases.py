@@ -1,0 +1,417 @@
+"""Performance cases of the quantized linear path: the projections of one decoder
+layer, a sparse MoE block, and a single projection, each called as a serving
+program calls them.
+
+A ``layer`` case is what one decoder layer asks of this package at ``m`` rows:
+the packed q/k/v projection of the hidden states, the output projection of the
+attention result, and the gated MLP ``down(silu(gate(x)) * up(x))``.  Attention
+and the norms lie outside the package, so their results (the layer's inputs
+``x``, ``a`` and ``y``) are given.  Decode batches replay the layer from a HIP
+graph, as a decode loop does; prefill chunks call it directly.  ``tp`` is the
+tensor-parallel degree whose shard of the layer this rank holds.
+
+Sizes: Llama-3-8B (4096 / 14336, 1024 key/value columns) and Qwen2-7B (3584 /
+18944, 512), the widths of the tests (11008, 5120 / 13824, 8192 / 28672) and the
+Qwen3-MoE block (128 experts, 2048 / 768, top 8).
+"""
+
+import math
+
+import torch
+
+from kairyu_amd.graphs import HipGraphBackend
+from kairyu_amd.moe import BlockFp8ExpertMlp, GroupedBlockFp8Experts
+from kairyu_amd.quant.linear import AwqLinear, BlockFp8Linear, Fp8Linear, GptqLinear, Int8Linear
+from kairyu_amd.quant.packed import QuantLinearPack
+
+AWQ_ORDER = (0, 2, 4, 6, 1, 3, 5, 7)
+
+
+def _layer(name, scheme, m, hidden, inter, kv, *, tp=1, group=128, act_order=False, bias=False,
+           dtype="bf16", graph=False):
+    return {"name": name, "kind": "layer", "scheme": scheme, "m": m, "hidden": hidden,
+            "inter": inter, "kv": kv, "tp": tp, "group": group, "act_order": act_order,
+            "bias": bias, "dtype": dtype, "graph": graph}
+
+
+def _moe(name, m, hidden, inter, experts, top_k, *, dtype="bf16", graph=False):
+    return {"name": name, "kind": "moe", "m": m, "hidden": hidden, "inter": inter,
+            "experts": experts, "top_k": top_k, "dtype": dtype, "graph": graph}
+
+
+def listed():
+    return [
+        # one user's decode step, 4-bit weights: pure weight streaming and launch latency
+        _layer("awq_decode_1", "awq", 1, 4096, 14336, 1024, dtype="fp16", graph=True),
+        # a small decode batch on an act-order checkpoint (activations gathered per call)
+        _layer("gptq_actorder_decode_16", "gptq", 16, 3584, 18944, 512, act_order=True, bias=True,
+               graph=True),
+        # a busy server's decode batch, past the GEMV's sixteen rows
+        _layer("awq_decode_48", "awq", 48, 4096, 14336, 1024, dtype="fp16", graph=True),
+        # a prompt of ragged length on 4-bit weights
+        _layer("awq_prefill_777", "awq", 777, 4096, 11008, 4096, dtype="fp16"),
+        # 8-bit decode, small batch
+        _layer("fp8_decode_8", "fp8", 8, 4096, 14336, 1024, graph=True),
+        # 8-bit integer decode, batch between two kernels' home ranges
+        _layer("int8_decode_24", "int8", 24, 3584, 18944, 512, bias=True, graph=True),
+        # a short prompt, or a chunk of one mixed with decode rows
+        _layer("int8_prefill_200", "int8", 200, 3584, 18944, 512, bias=True),
+        # a full prefill batch: the matrix cores' case
+        _layer("fp8_prefill_4096", "fp8", 4096, 4096, 14336, 1024),
+        # block-scaled checkpoint, small decode batch
+        _layer("block_fp8_decode_8", "fp8_block", 8, 4096, 12288, 1024, graph=True),
+        # MoE decode: few tokens, most of the touched experts hold one or two rows
+        _moe("moe_decode_16", 16, 2048, 768, 128, 8, graph=True),
+        # MoE prefill: every expert holds a few hundred rows
+        _moe("moe_prefill_4096", 4096, 2048, 768, 128, 8),
+        # the smallest call: one narrow projection, statically scaled, called directly
+        {"name": "fp8_linear_5", "kind": "linear", "scheme": "fp8", "m": 5, "k": 4096, "n": 1024,
+         "bias": True, "static": True, "dtype": "bf16", "graph": False},
+    ]
+
+
+WIDTHS = ((4096, 14336, 1024), (3584, 18944, 512), (4096, 11008, 4096), (5120, 13824, 1024),
+          (8192, 28672, 1024), (2048, 6144, 512), (4096, 12288, 1024))
+
+
+def _cost(case):
+    """Seconds a pass might take, for keeping a drawn case below the largest listed one."""
+    w = work(case)
+    rate = 1e15 if case.get("scheme") in ("awq", "gptq", None) else 2e15
+    return w["flops"] / rate + w["bytes"] / 4e12
+
+
+def _log_int(rng, low, high):
+    return min(high, max(low, round(math.exp(rng.uniform(math.log(low), math.log(high))))))
+
+
+def draw(rng):
+    most = max(_cost(c) for c in listed())
+    kind = rng.choices(("layer", "moe", "linear"), (8, 2, 1))[0]
+    m = _log_int(rng, 1, 4096)
+    dtype = rng.choice(("bf16", "bf16", "fp16"))
+    graph = m <= 64 and rng.random() < 0.8
+    if kind == "moe":
+        hidden, inter, experts, top_k = rng.choice(
+            ((2048, 768, 128, 8), (2048, 1024, 64, 8), (4096, 1536, 64, 8), (1024, 512, 32, 4)))
+        case = _moe("", m, hidden, inter, experts, top_k, dtype=dtype, graph=graph)
+    elif kind == "linear":
+        case = {"kind": "linear", "scheme": rng.choice(("fp8", "int8", "awq", "gptq", "fp8_block")),
+                "m": m, "k": 128 * _log_int(rng, 4, 96), "n": 16 * _log_int(rng, 16, 1024),
+                "bias": rng.random() < 0.5, "static": rng.random() < 0.3, "dtype": dtype,
+                "graph": graph}
+    else:
+        scheme = rng.choice(("awq", "gptq", "fp8", "int8", "fp8_block"))
+        hidden, inter, kv = rng.choice(WIDTHS)
+        tp = rng.choice((1, 1, 2, 4, 8))
+        group = rng.choice((128, 128, 64, 32))
+        if scheme == "fp8_block":  # shards of whole 128-wide blocks
+            while hidden // tp % 128 or inter // tp % 128:
+                tp //= 2
+        while any(k % group for k in (hidden, hidden // tp, inter // tp)):
+            group //= 2
+        case = _layer("", scheme, m, hidden, inter, kv, tp=tp, group=group,
+                      act_order=scheme == "gptq" and rng.random() < 0.5, bias=rng.random() < 0.3,
+                      dtype=dtype, graph=graph)
+    case.pop("name", None)
+    while _cost(case) > most and case["m"] > 1:
+        case["m"] = max(1, case["m"] * 2 // 3)
+    return case
+
+
+# ------------------------------------------------------------------- shapes
+def _projections(case):
+    """(name, K, N, biased) of a layer's projections on this rank, in call order."""
+    h, i, kv, tp = case["hidden"], case["inter"], case["kv"], case["tp"]
+    return [("q", h, h // tp, case["bias"]), ("k", h, kv // tp, case["bias"]),
+            ("v", h, kv // tp, case["bias"]), ("o", h // tp, h, False),
+            ("gate", h, i // tp, False), ("up", h, i // tp, False), ("down", i // tp, h, False)]
+
+
+def _weight_bytes(scheme, k, n, group, act_order):
+    if scheme in ("awq", "gptq"):
+        groups = -(-k // group)
+        return k * n // 2 + groups * n // 2 + groups * n * 2 + (4 * k if act_order else 0)
+    if scheme == "fp8_block":
+        return k * n + 4 * -(-k // 128) * -(-n // 128)
+    return k * n + 4 * n
+
+
+def work(case):
+    m = case["m"]
+    if case["kind"] == "moe":
+        h, i, e, top_k = case["hidden"], case["inter"], case["experts"], case["top_k"]
+        expert = 3 * i * h * (1 + 4 / 16384)
+        touched = e * (1.0 - (1.0 - top_k / e) ** m)  # each token takes top_k distinct experts
+        return {"bytes": touched * expert + 2 * m * h * 2 + m * e * 4 + m * top_k * 8,
+                "flops": 2.0 * m * top_k * 3 * i * h}
+    if case["kind"] == "linear":
+        k, n = case["k"], case["n"]
+        return {"bytes": _weight_bytes(case["scheme"], k, n, 128, False) + 2 * m * (k + n)
+                + (2 * n if case["bias"] else 0), "flops": 2.0 * m * n * k}
+    sizes = _projections(case)
+    weights = sum(_weight_bytes(case["scheme"], k, n, case["group"], case["act_order"])
+                  + (2 * n if b else 0) for _, k, n, b in sizes)
+    by = {name: (k, n) for name, k, n, _ in sizes}
+    rows = 2 * case["hidden"] + by["o"][0] + sum(by[p][1] for p in ("q", "k", "v", "o", "down"))
+    return {"bytes": weights + 2 * m * rows, "flops": 2.0 * m * sum(k * n for _, k, n, _ in sizes)}
+
+
+# ------------------------------------------------------------------- inputs
+def _dtype(case):
+    return torch.float16 if case["dtype"] == "fp16" else torch.bfloat16
+
+
+def _gen(seed):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    return g
+
+
+def _rows(g, m, k, dtype):
+    """Activations N(0, 1) with one channel value in a hundred twenty times as large."""
+    x = torch.randn((m, k), generator=g, device="cuda")
+    large = torch.rand((m, k), generator=g, device="cuda") < 0.01
+    return torch.where(large, x * 20.0, x).to(dtype)
+
+
+def _weight(g, scheme, k, n, group, g_idx, bias, dtype):
+    """The tensors of one projection's checkpoint, as a dict."""
+    w = {}
+    if scheme in ("awq", "gptq"):
+        groups = -(-k // group)
+        w["q"] = torch.randint(0, 16, (k, n), generator=g, device="cuda", dtype=torch.int32)
+        # AWQ zeros vary around the middle; GPTQ checkpoints are symmetric (z = 8)
+        w["z"] = (torch.randint(5, 12, (groups, n), generator=g, device="cuda", dtype=torch.int32)
+                  if scheme == "awq" else torch.full((groups, n), 8, device="cuda", dtype=torch.int32))
+        w["s"] = (torch.rand((groups, n), generator=g, device="cuda") * 0.009 + 0.001).half()
+        w["g_idx"] = g_idx
+    else:
+        f = torch.randn((n, k), generator=g, device="cuda") * 0.02
+        if scheme == "fp8_block":
+            nb, kb = -(-n // 128), -(-k // 128)
+            pad = torch.zeros((nb * 128, kb * 128), device="cuda")
+            pad[:n, :k] = f
+            w["s"] = pad.view(nb, 128, kb, 128).abs().amax(dim=(1, 3)).clamp(min=1e-12) / 448.0
+            wide = w["s"].repeat_interleave(128, 0).repeat_interleave(128, 1)[:n, :k]
+            w["w"] = (f / wide).clamp(-448.0, 448.0).to(torch.float8_e4m3fn)
+        elif scheme == "fp8":
+            w["s"] = f.abs().amax(dim=1, keepdim=True).clamp(min=1e-12) / 448.0
+            w["w"] = (f / w["s"]).clamp(-448.0, 448.0).to(torch.float8_e4m3fn)
+        else:
+            w["s"] = f.abs().amax(dim=1, keepdim=True).clamp(min=1e-12) / 127.0
+            w["w"] = torch.round(f / w["s"]).clamp(-127, 127).to(torch.int8)
+    w["bias"] = torch.randn((n,), generator=g, device="cuda").mul_(0.1).to(dtype) if bias else None
+    return w
+
+
+def _g_idx(g, case, k):
+    if case.get("act_order"):
+        return (torch.randperm(k, generator=g, device="cuda") // case["group"]).to(torch.int32)
+    return (torch.arange(k, device="cuda") // case.get("group", 128)).to(torch.int32)
+
+
+def _inputs(case, seed):
+    g, m, dtype = _gen(seed), case["m"], _dtype(case)
+    if case["kind"] == "moe":
+        h, i, e = case["hidden"], case["inter"], case["experts"]
+        def stack(n, k):
+            f = torch.randn((e, n // 128, 128, k // 128, 128), generator=g, device="cuda") * 0.02
+            s = f.abs().amax(dim=(2, 4)).clamp(min=1e-12) / 448.0
+            q = (f / s[:, :, None, :, None]).clamp(-448.0, 448.0).to(torch.float8_e4m3fn)
+            return q.view(e, n, k), s
+        w13, s13 = stack(2 * i, h)
+        w2, s2 = stack(h, i)
+        x = torch.randn((m, h), generator=g, device="cuda").to(dtype)
+        logits = torch.randn((m, e), generator=g, device="cuda")
+        return {"w13": w13, "s13": s13, "w2": w2, "s2": s2, "x": x, "logits": logits}
+    if case["kind"] == "linear":
+        k, n = case["k"], case["n"]
+        d = {"x": _rows(g, m, k, dtype),
+             "w": _weight(g, case["scheme"], k, n, 128, _g_idx(g, case, k), case["bias"], dtype)}
+        # a calibrated per-tensor scale: the largest value the rows are expected to hold
+        d["input_scale"] = (torch.full((1,), 80.0 / 448.0, device="cuda")
+                            if case["static"] and case["scheme"] == "fp8" else None)
+        return d
+    d = {"x": _rows(g, m, case["hidden"], dtype), "y": _rows(g, m, case["hidden"], dtype),
+         "a": torch.randn((m, case["hidden"] // case["tp"]), generator=g, device="cuda").to(dtype)}
+    order = {}
+    for name, k, n, bias in _projections(case):
+        # projections of one input share its act-order
+        source = {"q": "x", "k": "x", "v": "x", "gate": "y", "up": "y"}.get(name, name)
+        if source not in order:
+            order[source] = _g_idx(g, case, k)
+        d[name] = _weight(g, case["scheme"], k, n, case["group"], order[source], bias, dtype)
+    return d
+
+
+# ------------------------------------------------------------------ modules
+def _pack_words(q, axis, order=range(8)):
+    """Eight nibbles along `axis` to one int32 word, nibble `i` from position order[i]."""
+    q = q.movedim(axis, -1)
+    q = q.reshape(*q.shape[:-1], q.shape[-1] // 8, 8)
+    words = torch.zeros(q.shape[:-1], dtype=torch.int32, device=q.device)
+    for nibble, position in enumerate(order):
+        words |= q[..., position] << (4 * nibble)
+    return words.movedim(-1, axis).contiguous()
+
+
+def _module(scheme, w, k, n, group, input_scale=None):
+    bias = w["bias"] is not None
+    if scheme == "awq":
+        module = AwqLinear(k, n, bias, group_size=group)
+        named = {"qweight": _pack_words(w["q"], 1, AWQ_ORDER), "scales": w["s"],
+                 "qzeros": _pack_words(w["z"], 1, AWQ_ORDER)}
+    elif scheme == "gptq":
+        module = GptqLinear(k, n, bias, group_size=group)
+        named = {"qweight": _pack_words(w["q"], 0), "qzeros": _pack_words(w["z"] - 1, 1),
+                 "scales": w["s"], "g_idx": w["g_idx"]}
+    elif scheme == "fp8":
+        module = Fp8Linear(k, n, bias, activation_dynamic=input_scale is None)
+        named = {"weight": w["w"], "weight_scale": w["s"]}
+        if input_scale is not None:
+            named["input_scale"] = input_scale
+    elif scheme == "int8":
+        module = Int8Linear(k, n, bias)
+        named = {"weight": w["w"], "weight_scale": w["s"]}
+    else:
+        module = BlockFp8Linear(k, n, bias)
+        named = {"weight": w["w"], "weight_scale_inv": w["s"]}
+    module = module.to("cuda")
+    with torch.no_grad():
+        for name, t in named.items():
+            getattr(module, name).copy_(t.reshape(getattr(module, name).shape))
+        if bias:
+            module.bias = torch.nn.Parameter(w["bias"].clone(), requires_grad=False)
+    return module
+
+
+def _step(case, d):
+    """The call of one pass, a function of the rows that arrive."""
+    if case["kind"] == "moe":
+        experts = GroupedBlockFp8Experts.from_tensors(d["w13"], d["s13"], d["w2"], d["s2"])
+        logits, top_k = d["logits"], case["top_k"]
+        return lambda x: experts.forward_logits(x, logits, top_k)
+    if case["kind"] == "linear":
+        return _module(case["scheme"], d["w"], case["k"], case["n"], 128, d["input_scale"])
+    mods = {name: _module(case["scheme"], d[name], k, n, case["group"])
+            for name, k, n, _ in _projections(case)}
+    attn, mlp_in, o, down = d["a"], d["y"], mods["o"], mods["down"]
+    if case["scheme"] == "fp8_block":
+        q, k, v = mods["q"], mods["k"], mods["v"]
+        mlp = BlockFp8ExpertMlp(128, 128)
+        mlp.gate_proj, mlp.up_proj, mlp.down_proj = mods["gate"], mods["up"], down
+        return lambda x: (q(x), k(x), v(x), o(attn), mlp(mlp_in))
+    qkv = QuantLinearPack.create([mods["q"], mods["k"], mods["v"]])
+    gate_up = QuantLinearPack.create([mods["gate"], mods["up"]])
+
+    def step(x):
+        q, k, v = qkv(x)
+        return q, k, v, o(attn), down(gate_up.swiglu(mlp_in))
+
+    return step
+
+
+def prepare(case, seed):
+    d = _inputs(case, seed)
+    with torch.no_grad():
+        step = _step(case, d)
+        if case["graph"]:
+            # the graph holds addresses alone: the layer's weights and inputs live as long as it does
+            graph = HipGraphBackend(warmup_iters=1).capture(step, d["x"])
+            return {"graph": graph, "step": step, "inputs": d}
+        step(d["x"])  # a serving program runs its layers once before the first request
+    return {"step": step, "x": d["x"]}
+
+
+def run(state):
+    if "graph" in state:
+        return state["graph"].replay()
+    with torch.no_grad():
+        return state["step"](state["x"])
+
+
+# ------------------------------------------------------------ 64-bit answers
+def _linear64(scheme, x, w, group, input_scale=None):
+    """One projection with its sums in 64 bits.  What the format itself rounds
+    (weights to fp16, activations to 8 bits with fp32 scales) is rounded here too."""
+    if scheme in ("awq", "gptq"):
+        which = w["g_idx"].long() if scheme == "gptq" else torch.arange(x.shape[1], device="cuda") // group
+        weight = ((w["q"] - w["z"][which]).float() * w["s"][which].float()).half().double()
+        out = x.float().clamp(-65504.0, 65504.0).half().double() @ weight
+    elif scheme == "fp8_block":
+        m, k = x.shape
+        blocks = x.float().view(m, k // 128, 128)
+        s = blocks.abs().amax(dim=2, keepdim=True).clamp(min=1e-12) / 448.0
+        q = (blocks / s).clamp(-448.0, 448.0).to(torch.float8_e4m3fn)
+        n = w["w"].shape[0]
+        wide = w["s"].double().repeat_interleave(128, 0).repeat_interleave(128, 1)[:n, :k]
+        out = (q.double() * s.double()).view(m, k) @ (w["w"].double() * wide).t()
+    else:
+        f = x.float()
+        most = 448.0 if scheme == "fp8" else 127.0
+        s = f.abs().amax(dim=1, keepdim=True).clamp(min=1e-12) / most
+        if input_scale is not None:
+            s = input_scale.reshape(1, 1)
+        q = f / s
+        q = (q.clamp(-most, most).to(torch.float8_e4m3fn) if scheme == "fp8"
+             else torch.round(q).clamp(-most, most)).double()
+        out = (q @ w["w"].double().t()) * s.double() * w["s"].double().reshape(1, -1)
+    return out if w["bias"] is None else out + w["bias"].double()
+
+
+def _swiglu64(gate, up, dtype):
+    """silu(gate) * up of tensors handed over in the activations' type."""
+    gate, up = gate.to(dtype).double(), up.to(dtype).double()
+    act = (gate / (1.0 + torch.exp(-gate))).to(dtype).double()
+    return (act * up).to(dtype)
+
+
+def _moe64(case, d):
+    top_k, dtype, x = case["top_k"], _dtype(case), d["x"]
+    index = torch.argsort(d["logits"], dim=1, descending=True, stable=True)[:, :top_k]
+    weight = torch.softmax(d["logits"].gather(1, index).double(), dim=1)
+    out = torch.zeros(x.shape, dtype=torch.float64, device="cuda")
+    inter = case["inter"]
+    for e in range(case["experts"]):
+        token, slot = (index == e).nonzero(as_tuple=True)
+        if token.numel() == 0:
+            continue
+        both = _linear64("fp8_block", x[token], {"w": d["w13"][e], "s": d["s13"][e], "bias": None}, 128)
+        act = _swiglu64(both[:, :inter], both[:, inter:], dtype)
+        y = _linear64("fp8_block", act, {"w": d["w2"][e], "s": d["s2"][e], "bias": None}, 128)
+        out.index_add_(0, token, y.to(dtype).double() * weight[token, slot].unsqueeze(1))
+    return out, index.int(), weight
+
+
+def exact(case, seed):
+    with torch.no_grad():
+        d = _inputs(case, seed)
+        if case["kind"] == "moe":
+            return _moe64(case, d)
+        scheme = case["scheme"]
+        if case["kind"] == "linear":
+            return _linear64(scheme, d["x"], d["w"], 128, d["input_scale"])
+        group = case["group"]
+        q, k, v = (_linear64(scheme, d["x"], d[p], group) for p in ("q", "k", "v"))
+        o = _linear64(scheme, d["a"], d["o"], group)
+        gate, up = (_linear64(scheme, d["y"], d[p], group) for p in ("gate", "up"))
+        down = _linear64(scheme, _swiglu64(gate, up, _dtype(case)), d["down"], group)
+        return q, k, v, o, down
+
+
+def tolerance(case):
+    """About four times the distance of one correct result from another.
+
+    4-bit weights and int8: sums agree but for their last bits, so what is left is
+    the rounding of the results (measured against `exact`: 1.7e-3 in bf16, 2.1e-4 in
+    fp16).  8-bit floats: the matrix cores' own sums of e4m3 products stand 2e-3 to
+    3e-3 from the exact ones, and where such a result is quantized again (the MLP's
+    activations, an expert's) values near a boundary of the 3-bit mantissa fall to the
+    other side: 3e-3 to 1.1e-2 after a dense MLP, 1.5e-2 after the experts.
+    """
+    if case["kind"] == "moe" or case["kind"] == "layer" and case["scheme"] in ("fp8", "fp8_block"):
+        return {"rel": 3e-2}
+    if case["scheme"] in ("fp8", "fp8_block"):
+        return {"rel": 1.2e-2}
+    return {"rel": 7e-3 if case["dtype"] == "bf16" else 1e-3}
