@@ -102,7 +102,8 @@ def draw(rng):
                 "graph": graph}
     else:
         scheme = rng.choice(("awq", "gptq", "fp8", "int8", "fp8_block"))
-        hidden, inter, kv = rng.choice(WIDTHS)
+        # block scaling takes projections of up to 16384 inputs
+        hidden, inter, kv = rng.choice([w for w in WIDTHS if scheme != "fp8_block" or w[1] <= 16384])
         tp = rng.choice((1, 1, 2, 4, 8))
         group = rng.choice((128, 128, 64, 32))
         if scheme == "fp8_block":  # shards of whole 128-wide blocks
