@@ -234,12 +234,10 @@ def gemm_launcher(workload, copies: int):
                          _native.stream_handle(device))
 
     nbytes = n * k + 4 * n + m * k + 4 * m + 2 * m * n
-    # the launcher's dispatch in kq_w8a8.hip: decode kernel for M <= 16 with
-    # K % 128 == 0, skinny kernel up to M = 64, tile engine above
-    if m <= 16 and k % 128 == 0:
-        kernel = "w8a8_decode_kernel"
-    elif m <= 64:
-        kernel = "w8a8_skinny_kernel (+ split-K reduce when used)"
+    # the launcher's dispatch in kq_w8a8.hip: the weight-streaming kernel up
+    # to M = 64, tile engine above
+    if m <= 64:
+        kernel = "stream_gemm_kernel"
     else:
         kernel = "tile_gemm_kernel (+ split-K reduce when used)"
     return launch, nbytes, 2 * m * n * k, kernel

@@ -122,7 +122,7 @@ size_t kq_w8a8_linear_workspace_size(int64_t m, int64_t n, int64_t k);
  * column c and up column i_width + c, with the roundings of
  * kq_w8a8_*_linear followed by kq_swiglu (bit-identical to that pair).
  * Prefill shapes apply SwiGLU in the tile engine's epilogue and shapes of
- * m <= 64 in the decode or skinny GEMM's (or the reduce of their K splits):
+ * m <= 64 in the weight-streaming GEMM's:
  * the [m][2I] projection never reaches memory; other shapes run the pair
  * through the workspace.  Replaces the reference MLP's act_fn(gate(x)) *
  * up(x) (kairyu/models/layers.py:243-244) over its packed projections
@@ -314,6 +314,27 @@ int kq_act_quant_fp8_blocks(const void* x, int x_dtype, int64_t rows, int64_t k,
 int kq_block_fp8_gemm(const uint8_t* xq, const float* xs, const uint8_t* w, const float* ws,
                       const void* bias, int bias_dtype, void* out, int out_dtype, int64_t m,
                       int64_t n, int64_t k, void* stream);
+
+/* kq_act_quant_fp8_blocks of x (fp16/bf16 [m, k], row pitch ldx) and
+ * kq_block_fp8_gemm in one call, out [m, n] in x_dtype: decode batches are
+ * quantized inside the GEMM launch, other shapes through the workspace
+ * (kq_block_fp8_workspace_size bytes).  Replaces finegrained_fp8_linear
+ * (deepseek_v4_moe_gpu.py:60-74) for BlockFp8Linear. */
+int kq_block_fp8_linear(const void* x, int x_dtype, int64_t ldx, const uint8_t* w, const float* ws,
+                        const void* bias, int bias_dtype, void* out, int64_t m, int64_t n, int64_t k,
+                        void* workspace, size_t workspace_bytes, void* stream);
+size_t kq_block_fp8_workspace_size(int64_t m, int64_t k);
+
+/* out [m, i_width] = silu(gate) * up of two block-FP8 projections [i_width, k]
+ * of the same x, m <= 64, with the roundings of the two linears followed by
+ * torch's silu and product (each projection's bias may be null, both of
+ * bias_dtype).  Replaces act_fn(gate(x)) * up(x) of the expert MLP
+ * (kairyu/models/moe.py:27-83). */
+int kq_block_fp8_swiglu_linear(const void* x, int x_dtype, int64_t ldx, const uint8_t* w_gate,
+                               const float* s_gate, const uint8_t* w_up, const float* s_up,
+                               const void* bias_gate, const void* bias_up, int bias_dtype, void* out,
+                               int64_t m, int64_t i_width, int64_t k, void* workspace,
+                               size_t workspace_bytes, void* stream);
 
 /* Qwen3 routing of logits [tokens, experts] (fp16/bf16/fp32; experts <= 512,
  * top_k <= 32): stable descending top-k (ties -> smaller expert id) into

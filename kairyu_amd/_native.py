@@ -81,6 +81,11 @@ _SIGNATURES: dict[str, list] = {
     "kq_moe_route_topk": [_P, _I, _I64, _I64, _I, _I, _P, _P, _P],
     "kq_act_quant_fp8_blocks": [_P, _I, _I64, _I64, _I64, _P, _P, _P],
     "kq_block_fp8_gemm": [_P, _P, _P, _P, _P, _I, _P, _I, _I64, _I64, _I64, _P],
+    "kq_block_fp8_linear": [_P, _I, _I64, _P, _P, _P, _I, _P, _I64, _I64, _I64, _P, _SZ, _P],
+    "kq_block_fp8_workspace_size": [_I64, _I64],
+    "kq_block_fp8_swiglu_linear": [
+        _P, _I, _I64, _P, _P, _P, _P, _P, _P, _I, _P, _I64, _I64, _I64, _P, _SZ, _P,
+    ],
     "kq_moe_workspace_size": [_I64, _I64, _I64, _I64, _I],
     "kq_peak_stream_read": [_P, _I64, _I, _P, _P],
     "kq_peak_mfma": [_I, _I64, _I, _P, _P],
@@ -121,6 +126,7 @@ def _load() -> ctypes.CDLL:
                           "kq_w8a8_workspace_size": ctypes.c_size_t,
                           "kq_w8a8_linear_workspace_size": ctypes.c_size_t,
                           "kq_w8a8_swiglu_workspace_size": ctypes.c_size_t,
+                          "kq_block_fp8_workspace_size": ctypes.c_size_t,
                           "kq_moe_workspace_size": ctypes.c_size_t}.get(name, ctypes.c_int)
         _lib = lib
         return lib

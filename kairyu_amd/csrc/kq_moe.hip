@@ -945,31 +945,6 @@ extern "C" int kq_act_quant_fp8_blocks(const void* x, int x_dtype, int64_t rows,
   return check_launch("kq_act_quant_fp8_blocks");
 }
 
-extern "C" int kq_block_fp8_gemm(const uint8_t* xq, const float* xs, const uint8_t* w,
-                                 const float* ws, const void* bias, int bias_dtype, void* out,
-                                 int out_dtype, int64_t m, int64_t n, int64_t k, void* stream) {
-  if (!quant_dtype_ok(out_dtype)) {
-    set_error("kq_block_fp8_gemm: output dtype must be fp16 or bf16");
-    return KQ_EUNSUPPORTED;
-  }
-  if (m < 0 || n < 1 || k < kTgBK || (k % kTgBK) != 0 || k > kTgBK * kTgMaxKB || m > 0x7fffffffLL ||
-      n > 0x7fffffffLL || n * k > 0x7fffffffLL || m * k > 0x7fffffffLL) {
-    set_error("kq_block_fp8_gemm: bad shape m=%lld n=%lld k=%lld (k must be a multiple of 128)",
-              (long long)m, (long long)n, (long long)k);
-    return KQ_EINVAL;
-  }
-  if (m == 0) return KQ_OK;
-  TileGemmArgs a{};
-  a.x = xq; a.xs = xs; a.x_rows = (int)m; a.gather = nullptr;
-  a.w = w; a.ws = ws; a.mtile_table = nullptr; a.mtile_count = nullptr;
-  a.M = (int)m; a.N = (int)n; a.K = (int)k; a.I = 0;
-  a.mtiles = (int)((m + kTgBM - 1) / kTgBM);
-  a.ntiles = (int)((n + kTgBN - 1) / kTgBN);
-  a.out = out; a.out_dtype = out_dtype; a.bias = bias; a.bias_dtype = bias_dtype;
-  tg_launch<kTgFp8, true, kTgEpiStore>(a, (hipStream_t)stream);
-  return check_launch("kq_block_fp8_gemm");
-}
-
 extern "C" size_t kq_moe_workspace_size(int64_t tokens, int64_t hidden, int64_t inter,
                                         int64_t experts, int top_k) {
   if (tokens < 1 || hidden < 1 || inter < 1 || experts < 1 || top_k < 1) return 0;

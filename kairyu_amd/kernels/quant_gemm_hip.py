@@ -508,15 +508,46 @@ def block_fp8_linear_forward(x: torch.Tensor, module, *, add_bias: bool = True) 
     if k % 128 != 0:
         raise ValueError(f"block FP8 kernel needs in_features % 128 == 0, got {k}")
     bias = _bias(module, add_bias)
-    x_q, x_scale = quantize_activation_blocks(flat)
     scale_inv = _f32(module.weight_scale_inv)
+    ws = _block_fp8_workspace(x.device, m, k)
     _native.call(
-        "kq_block_fp8_gemm", x_q.data_ptr(), x_scale.data_ptr(), module.weight.data_ptr(),
-        scale_inv.data_ptr(), _native.ptr(bias),
-        _native.dtype_code(None if bias is None else bias.dtype), out.data_ptr(),
-        _native.dtype_code(out.dtype), m, module.out_features, k, _native.stream_handle(x.device),
+        "kq_block_fp8_linear", flat.data_ptr(), _native.dtype_code(flat.dtype), flat.stride(0),
+        module.weight.data_ptr(), scale_inv.data_ptr(), _native.ptr(bias),
+        _native.dtype_code(None if bias is None else bias.dtype), out.data_ptr(), m,
+        module.out_features, k, ws.data_ptr(), ws.numel(), _native.stream_handle(x.device),
     )
     return out.reshape(*x.shape[:-1], module.out_features)
+
+
+def _block_fp8_workspace(device: torch.device, m: int, k: int) -> torch.Tensor:
+    need = _workspace_bytes("kq_block_fp8_workspace_size", _device_index(device), m, k)
+    return _workspace(device, need)
+
+
+BLOCK_SWIGLU_ROWS = 64
+
+
+def block_fp8_swiglu_forward(x: torch.Tensor, gate, up) -> torch.Tensor:
+    """``silu(gate(x)) * up(x)`` of two block-FP8 projections of one input, at
+    most ``BLOCK_SWIGLU_ROWS`` rows, in one GEMM launch with torch's roundings."""
+
+    flat, out = _prepare(x, gate, "fp8_block")
+    _prepare(x, up, "fp8_block", allocate_output=False)
+    m, k = flat.shape
+    if k % 128 != 0:
+        raise ValueError(f"block FP8 kernel needs in_features % 128 == 0, got {k}")
+    bias = _bias(gate, gate._add_local_bias())
+    bias_up = _bias(up, up._add_local_bias())
+    scales, scales_up = _f32(gate.weight_scale_inv), _f32(up.weight_scale_inv)
+    ws = _block_fp8_workspace(x.device, m, k)
+    _native.call(
+        "kq_block_fp8_swiglu_linear", flat.data_ptr(), _native.dtype_code(flat.dtype), flat.stride(0),
+        gate.weight.data_ptr(), scales.data_ptr(), up.weight.data_ptr(), scales_up.data_ptr(),
+        _native.ptr(bias), _native.ptr(bias_up), _native.dtype_code(None if bias is None else bias.dtype),
+        out.data_ptr(), m, gate.out_features, k, ws.data_ptr(), ws.numel(),
+        _native.stream_handle(x.device),
+    )
+    return out.reshape(*x.shape[:-1], gate.out_features)
 
 
 _DISPATCH = {

@@ -33,6 +33,7 @@ from kairyu_amd.quant.linear import (
     ModelScope,
     make_linear,
 )
+from kairyu_amd.quant.packed import _plain
 
 __all__ = [
     "BlockFp8ExpertMlp",
@@ -132,7 +133,33 @@ class BlockFp8ExpertMlp(nn.Module):
                                      shard_dim=1, **common)
 
     def forward(self, hidden: torch.Tensor) -> torch.Tensor:
+        if hidden.is_cuda and self._fused_swiglu(hidden):
+            from kairyu_amd.kernels import quant_gemm_hip as hip
+
+            return self.down_proj(hip.block_fp8_swiglu_forward(hidden, self.gate_proj, self.up_proj))
         return self.down_proj(nn.functional.silu(self.gate_proj(hidden)) * self.up_proj(hidden))
+
+    def _fused_swiglu(self, hidden: torch.Tensor) -> bool:
+        """Whether gate, up and their SwiGLU run as one launch: a decode batch
+        through two plain block-FP8 projections (no hooks, no other forward
+        bound) of equal widths and alike biases."""
+
+        from kairyu_amd.kernels import quant_gemm_hip as hip
+
+        gate, up = self.gate_proj, self.up_proj
+        if not 0 < hidden.numel() <= hip.BLOCK_SWIGLU_ROWS * hidden.shape[-1]:
+            return False
+        for m in (gate, up):
+            if type(m) is not BlockFp8Linear or not _plain(m):
+                return False
+            if getattr(m, "_fused_forward", None) not in (None, hip.block_fp8_linear_forward):
+                return False
+        biases = [m.bias if m._add_local_bias() else None for m in (gate, up)]
+        if (biases[0] is None) != (biases[1] is None):
+            return False
+        if biases[0] is not None and biases[0].dtype != biases[1].dtype:
+            return False
+        return (gate.in_features, gate.out_features) == (up.in_features, up.out_features)
 
 
 class GroupedBlockFp8Experts:

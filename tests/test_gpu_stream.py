@@ -1,0 +1,126 @@
+"""The weight-streaming GEMM (at most 64 rows) at the edges of its forms: row
+tiles of 16, 32, 48 and 64, a weight tile or two per workgroup, 4 to 16 waves,
+K blocks fewer than the waves, K tails, ragged columns."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_helpers import banner, bits, check_block_fp8, check_fp8, np32
+from kairyu_amd.kernels import quant_gemm_hip as hip
+from kairyu_amd.moe import BlockFp8ExpertMlp
+from kairyu_amd.quant.block_fp8 import quantize_block_fp8
+from kairyu_amd.quant.fp8 import quantize_fp8
+from kairyu_amd.quant.int8 import quantize_int8_weight
+from kairyu_amd.quant.linear import BlockFp8Linear, Fp8Linear, Int8Linear
+from oracle import linear as olinear
+
+pytestmark = pytest.mark.gpu
+
+ROWS = [1, 2, 15, 16, 17, 32, 33, 48, 49, 64]
+# one block, a tail of 16 bytes, 19 blocks for 16 waves with a tail; 1 to 600
+# column tiles (16 waves, 8 waves, two tiles, many workgroups per CU)
+SHAPES = [(24, 112), (200, 144), (2600, 2368), (4616, 640), (9608, 272)]
+
+
+def _gen(seed):
+    return torch.Generator().manual_seed(seed)
+
+
+def _fill(module, g):
+    w = torch.randn(module.out_features, module.in_features, generator=g) * 0.05
+    quantize = {Fp8Linear: quantize_fp8, Int8Linear: quantize_int8_weight, BlockFp8Linear: quantize_block_fp8}
+    q, s = quantize[type(module)](w)
+    module.weight.copy_(q)
+    (module.weight_scale_inv if isinstance(module, BlockFp8Linear) else module.weight_scale).copy_(s)
+    if module.bias is not None:
+        module.bias.data.normal_(generator=g)
+    return module
+
+
+@pytest.mark.parametrize("n,k", SHAPES)
+def test_int8_rows_are_exact(cuda, n, k):
+    module = _fill(Int8Linear(k, n, True), _gen(n + k)).to(cuda)
+    for m in ROWS:
+        banner(f"stream int8 m={m} n={n} k={k}")
+        x = torch.randn(m, k, generator=_gen(m)).to(torch.bfloat16)
+        acc = torch.empty(m, n, dtype=torch.int32, device=cuda)
+        out = hip.int8_linear_forward(x.to(cuda), module, accumulators=acc)
+        want, _, _, want_acc = olinear.int8_forward(
+            np32(x), module.weight.cpu().numpy(), module.weight_scale.cpu().numpy(), np32(module.bias))
+        assert np.array_equal(acc.cpu().numpy().astype(np.int64), want_acc)
+        assert np.array_equal(np32(out), want)
+
+
+@pytest.mark.parametrize("n,k", SHAPES)
+def test_fp8_rows_match_oracle(cuda, n, k):
+    module = _fill(Fp8Linear(k, n, True), _gen(n + k)).to(cuda)
+    for m in ROWS:
+        banner(f"stream fp8 m={m} n={n} k={k}")
+        x = torch.randn(m, k, generator=_gen(m)).to(torch.float16)
+        check_fp8(module(x.to(cuda)), x, module, label=f"m={m} n={n} k={k}")
+
+
+# 16 rows quantize in the launch up to K = 8192; 129 blocks would not fit
+@pytest.mark.parametrize("n,k", [(24, 128), (200, 384), (2600, 2432), (4616, 640), (9608, 256), (72, 16384)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_block_fp8_rows_match_oracle(cuda, n, k, dtype):
+    module = _fill(BlockFp8Linear(k, n, True), _gen(n + k)).to(cuda)
+    for m in [1, 8, 9] + ROWS[3:]:
+        banner(f"stream block fp8 m={m} n={n} k={k} {dtype}")
+        x = torch.randn(m, k, generator=_gen(m)).to(dtype)
+        x[0, :k // 2] = 0.0
+        check_block_fp8(module(x.to(cuda)), x, module, label=f"m={m} n={n} k={k}")
+
+
+@pytest.mark.parametrize("m", [1, 8, 16, 40, 64, 65])
+@pytest.mark.parametrize("n,k", [(200, 384), (5000, 256)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_block_fp8_mlp_matches_its_projections(cuda, m, n, k, bias):
+    """The expert MLP, whose gate, up and SwiGLU are one launch up to 64 rows,
+    against down(silu(gate(x)) * up(x)) of the same modules: the sums of a
+    gate or up column may be added in another order, so a rounding of the
+    activation dtype apart (2^-8 relative in bf16, from both factors)."""
+    mlp = BlockFp8ExpertMlp(128, 128)
+    g = _gen(m + n)
+    mlp.gate_proj, mlp.up_proj = (_fill(BlockFp8Linear(k, n, bias), g) for _ in range(2))
+    mlp.down_proj = torch.nn.Identity()
+    mlp = mlp.to(cuda)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(cuda)
+    banner(f"stream block swiglu m={m} n={n} k={k}")
+    out = mlp(x)
+    gate, up = mlp.gate_proj(x), mlp.up_proj(x)
+    want = torch.nn.functional.silu(gate) * up
+    torch.testing.assert_close(out.float(), want.float(), rtol=2.0 ** -6, atol=2.0 ** -9 * float(up.abs().max()))
+    if m == 65:  # past the launch's rows: the projections themselves
+        assert np.array_equal(bits(out), bits(want))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_block_fp8_launch_quantizes_as_the_quantizer(cuda, dtype):
+    """Edge values through the launch that quantizes and through the quantizer
+    and the GEMM: the same bits, NaN and infinite rows included."""
+    n, k, m = 200, 512, 8
+    module = _fill(BlockFp8Linear(k, n, False), _gen(5)).to(cuda)
+    x = torch.randn(m, k, generator=_gen(6)) * 5
+    x[0, :128:3] = -0.0
+    x[1, :128] = torch.tensor([1.0625, -1.1875, 0.017578125, 240.0]).repeat(32)
+    x[1, 127] = 448.0                      # scale 1: exact ties of e4m3
+    x[2, 128:256] = torch.randn(128, generator=_gen(7)) * 1e-30
+    x[3, 300] = float("inf")
+    x[4, 100] = float("nan")
+    x[5] = 0.0
+    x[6, 0] = 60000.0
+    x = x.to(dtype).to(cuda)
+    banner(f"stream block fp8 edge values {dtype}")
+    out = module(x)
+    q, s = hip.quantize_activation_blocks(x)
+    want = torch.empty_like(out)
+    hip._native.call("kq_block_fp8_gemm", q.data_ptr(), s.data_ptr(), module.weight.data_ptr(),
+                     module.weight_scale_inv.data_ptr(), None, hip._native.DTYPE_NONE, want.data_ptr(),
+                     hip._native.dtype_code(dtype), m, n, k, hip._native.stream_handle(cuda))
+    finite = [0, 1, 2, 5, 6, 7]
+    assert np.array_equal(bits(out)[finite], bits(want)[finite])
+    assert torch.equal(torch.isnan(out), torch.isnan(want))
