@@ -34,6 +34,7 @@
 // MFMA spans one 128-wide K block, and its fp32 result is scaled by
 // s_act[row][kb] * s_w[nb][kb] before it is added to the accumulator.
 #include "kq_common.h"
+#include "kq_stream_gemm.h"
 #include "kq_tile_gemm.h"
 
 #include <algorithm>
@@ -177,6 +178,26 @@ constexpr int kFusedScanMax = 32768;
 // 320-row one (measured 3-6% at 16 to 1024 tokens of the C5 layer).
 static inline int moe_nrb(int64_t routed_rows, int64_t experts) {
   return routed_rows > 192 * experts ? 5 : 4;
+}
+
+// Experts of few rows (decode batches): rows of the weight-streaming kernel's
+// row tiles, 0 where the tile engine runs.  The 256-row tiles stream 604 MB of
+// weights at C5's widths in 158 us whatever the rows, with one K block in
+// flight per CU; the streaming kernel's cost grows with its row tile, so that
+// is the smallest that holds nearly every expert's rows at an even routing
+// (a further tile reads the expert's weights again).  C5's widths, whole call
+// (graph replay; before, after): 16 tokens (8-row tiles) 116 -> 84 us, 32
+// (8) 157 -> 102, 64 (16) 159 -> 137, 128 (32) 161 -> 139, 256 (32) 165 ->
+// 152; 512 tokens take 174 us with 256-row tiles and 250 with 64-row ones.
+static inline int moe_stream_rows(int64_t routed_rows, int64_t experts) {
+  if (routed_rows <= 2 * experts) return 8;
+  if (routed_rows <= 6 * experts) return 16;
+  if (routed_rows <= 16 * experts) return 32;
+  return 0;
+}
+static inline int moe_tile_rows(int64_t routed_rows, int64_t experts) {
+  const int few = moe_stream_rows(routed_rows, experts);
+  return few ? few : 64 * moe_nrb(routed_rows, experts);
 }
 
 // Per-chunk expert histogram of the CR rows of chunk c: counts[c][e]
@@ -728,7 +749,7 @@ moe_combine_kernel(const uint16_t* __restrict__ y, int y_dtype, const int32_t* _
 
 // ------------------------------------------------------------------- host
 struct MoeWorkspace {
-  size_t counts, base, offsets, tiles, tile_count, sorted, inv, xq, xs, actq, acts, y, total;
+  size_t counts, base, offsets, tiles, tile_count, sorted, inv, xq, xs, act, actq, acts, y, total;
 };
 
 static size_t align256(size_t v) { return (v + 255) / 256 * 256; }
@@ -742,7 +763,7 @@ static MoeWorkspace moe_layout(int64_t T, int64_t H, int64_t I, int64_t E, int64
     const int64_t tpc = moe_routed_chunk_tokens(T, (int)k, E);
     C = std::max(C, (T + tpc - 1) / tpc);
   }
-  const int64_t BM = 64 * moe_nrb(R, E);
+  const int64_t BM = moe_tile_rows(R, E);
   const int64_t max_tiles = (R + BM - 1) / BM + E;
   MoeWorkspace w{};
   size_t p = 0;
@@ -756,6 +777,7 @@ static MoeWorkspace moe_layout(int64_t T, int64_t H, int64_t I, int64_t E, int64
   w.inv = take((size_t)R * 4);
   w.xq = take((size_t)T * H);
   w.xs = take((size_t)T * (H / 128) * 4);
+  w.act = take(moe_stream_rows(R, E) ? (size_t)R * I * 2 : 0);
   w.actq = take((size_t)R * I);
   w.acts = take((size_t)R * (I / 128) * 4);
   w.y = take((size_t)R * H * 2);
@@ -779,14 +801,14 @@ struct MoeCall {
   const void* hidden;
   int dtype, top_k;
   int64_t tokens, H, I, E;
-  int R, CR, C, nrb, BM, max_tiles, KY;
+  int R, CR, C, nrb, few, BM, max_tiles, KY;  // few: rows of a streaming kernel's tile, 0: tile engine
   int tpc;              // routed call: tokens per sort chunk (CR = tpc * top_k)
   int units;            // token quantization units (kQuantRows rows x one 2048-element span)
   bool vec;
   int32_t *counts, *base, *offsets, *tiles, *tile_count, *sorted, *inv;
   uint8_t *xq, *actq;
   float *xs, *acts;
-  uint16_t* y;
+  uint16_t *act, *y;
 };
 
 static MoeCall moe_call(const void* hidden, int dtype, int64_t tokens, int64_t H, int64_t I, int64_t E,
@@ -801,7 +823,8 @@ static MoeCall moe_call(const void* hidden, int dtype, int64_t tokens, int64_t H
   m.CR = routed ? m.tpc * top_k : moe_chunk_rows(top_k);
   m.C = (m.R + m.CR - 1) / m.CR;
   m.nrb = moe_nrb(m.R, E);
-  m.BM = 64 * m.nrb;
+  m.few = moe_stream_rows(m.R, E);
+  m.BM = moe_tile_rows(m.R, E);
   m.max_tiles = (m.R + m.BM - 1) / m.BM + (int)E;
   m.KY = (int)((H + 2047) / 2048);
   m.units = (int)((tokens + kQuantRows - 1) / kQuantRows) * m.KY;
@@ -815,10 +838,58 @@ static MoeCall moe_call(const void* hidden, int dtype, int64_t tokens, int64_t H
   m.inv = (int32_t*)(ws + L.inv);
   m.xq = ws + L.xq;
   m.xs = (float*)(ws + L.xs);
+  m.act = (uint16_t*)(ws + L.act);
   m.actq = ws + L.actq;
   m.acts = (float*)(ws + L.acts);
   m.y = (uint16_t*)(ws + L.y);
   return m;
+}
+
+// Both expert projections with the weight-streaming kernel: gate_up stores
+// silu(gate) * up in the activation dtype, and down quantizes it itself (row
+// tiles of 8 or 16) or after the block quantizer.  Workgroups are small (an
+// expert's projection is many), 2 waves of 2 or 4 column tiles: more waves
+// leave each one or two K blocks of down's few (C5 at 16 tokens, 2 waves and 2
+// tiles 84 us, 4 waves 91, 4 tiles 92; at 64 tokens 4 tiles 137, 2 tiles 159).
+static void moe_stream_gate_up(const MoeCall& m, const StreamArgs& a, hipStream_t st) {
+  constexpr int DT = KQ_DTYPE_BF16;  // (of no use to quantized rows)
+  if (m.few == 8) sg_launch_form<kSgBlock, false, 1, 2, 2, 3, 1, true, DT>(a, m.max_tiles, st);
+  else if (m.few == 16) sg_launch_form<kSgBlock, false, 1, 4, 2, 2, 1, true, DT>(a, m.max_tiles, st);
+  else sg_launch_form<kSgBlock, false, 2, 2, 2, 3, 1, true, DT>(a, m.max_tiles, st);
+}
+
+template <int DT>
+static void moe_stream_down_raw(const MoeCall& m, const StreamArgs& a, hipStream_t st) {
+  if (m.few == 8) sg_launch_form<kSgBlock, true, 1, 2, 2, 3, 1, false, DT>(a, m.max_tiles, st);
+  else sg_launch_form<kSgBlock, true, 1, 4, 2, 3, 2, false, DT>(a, m.max_tiles, st);
+}
+
+static void moe_stream_experts(const MoeCall& m, const uint8_t* w13, const float* s13, const uint8_t* w2,
+                               const float* s2, hipStream_t st) {
+  const int64_t HB = m.H / 128, IB = m.I / 128;
+  StreamArgs g{};
+  g.x = m.xq; g.x_bytes = (uint32_t)(m.tokens * m.H); g.xs = m.xs; g.x_rows = (int)m.tokens;
+  g.w = w13; g.w_up = w13 + m.I * m.H; g.w_pitch = 2 * m.I * m.H;
+  g.ws = s13; g.ws_up = s13 + IB * HB; g.ws_pitch = 2 * IB * HB;
+  g.gather = m.sorted; g.table = m.tiles; g.count = m.tile_count;
+  g.M = m.R; g.N = (int)m.I; g.K = (int)m.H;
+  g.bias_dtype = KQ_DTYPE_NONE; g.out = m.act; g.out_dtype = m.dtype;
+  moe_stream_gate_up(m, g, st);
+
+  StreamArgs d{};
+  d.w = w2; d.w_pitch = m.H * m.I; d.ws = s2; d.ws_pitch = HB * IB;
+  d.table = m.tiles; d.count = m.tile_count;
+  d.M = m.R; d.N = (int)m.H; d.K = (int)m.I;
+  d.bias_dtype = KQ_DTYPE_NONE; d.out = m.y; d.out_dtype = m.dtype;
+  if (m.few <= 16) {
+    d.x = m.act; d.ldx = (int)m.I; d.x_bytes = (uint32_t)((int64_t)m.R * m.I * 2);
+    if (m.dtype == KQ_DTYPE_BF16) moe_stream_down_raw<KQ_DTYPE_BF16>(m, d, st);
+    else moe_stream_down_raw<KQ_DTYPE_F16>(m, d, st);
+    return;
+  }
+  launch_act_quant_blocks(m.act, m.dtype, m.R, m.I, m.I, m.actq, m.acts, st);
+  d.x = m.actq; d.x_bytes = (uint32_t)((int64_t)m.R * m.I); d.xs = m.acts; d.x_rows = m.R;
+  sg_launch_form<kSgBlock, false, 2, 2, 2, 3, 1, false, KQ_DTYPE_BF16>(d, m.max_tiles, st);
 }
 
 // After the chunk histograms and the token quantization: the stable sort's
@@ -847,23 +918,27 @@ static void moe_sort_experts_combine(const MoeCall& m, const int32_t* topk_idx, 
                        topk_idx, m.R, m.CR, E, m.top_k, m.base, m.sorted, m.inv);
   }
 
-  TileGemmArgs g{};
-  g.x = m.xq; g.xs = m.xs; g.x_rows = (int)m.tokens; g.gather = m.sorted; g.gather_rows = m.R;
-  g.w = w13; g.ws = s13; g.mtile_table = m.tiles; g.mtile_count = m.tile_count;
-  g.N = (int)(2 * m.I); g.K = (int)m.H; g.I = (int)m.I;
-  g.mtiles = m.max_tiles; g.ntiles = (int)(m.I / 128);
-  g.actq = m.actq; g.acts = m.acts; g.out_dtype = m.dtype; g.bias_dtype = KQ_DTYPE_NONE;
-  if (m.nrb == 5) tg_launch<kTgFp8, true, kTgEpiSwiGluQuant, 5, true>(g, st);
-  else tg_launch<kTgFp8, true, kTgEpiSwiGluQuant, 4, true>(g, st);
+  if (m.few) {
+    moe_stream_experts(m, w13, s13, w2, s2, st);
+  } else {
+    TileGemmArgs g{};
+    g.x = m.xq; g.xs = m.xs; g.x_rows = (int)m.tokens; g.gather = m.sorted; g.gather_rows = m.R;
+    g.w = w13; g.ws = s13; g.mtile_table = m.tiles; g.mtile_count = m.tile_count;
+    g.N = (int)(2 * m.I); g.K = (int)m.H; g.I = (int)m.I;
+    g.mtiles = m.max_tiles; g.ntiles = (int)(m.I / 128);
+    g.actq = m.actq; g.acts = m.acts; g.out_dtype = m.dtype; g.bias_dtype = KQ_DTYPE_NONE;
+    if (m.nrb == 5) tg_launch<kTgFp8, true, kTgEpiSwiGluQuant, 5, true>(g, st);
+    else tg_launch<kTgFp8, true, kTgEpiSwiGluQuant, 4, true>(g, st);
 
-  TileGemmArgs d{};
-  d.x = m.actq; d.xs = m.acts; d.x_rows = m.R; d.gather = nullptr;
-  d.w = w2; d.ws = s2; d.mtile_table = m.tiles; d.mtile_count = m.tile_count;
-  d.N = (int)m.H; d.K = (int)m.I; d.I = 0;
-  d.mtiles = m.max_tiles; d.ntiles = (int)((m.H + kTgBN - 1) / kTgBN);
-  d.out = m.y; d.out_dtype = m.dtype; d.bias = nullptr; d.bias_dtype = KQ_DTYPE_NONE;
-  if (m.nrb == 5) tg_launch<kTgFp8, true, kTgEpiStore, 5, true>(d, st);
-  else tg_launch<kTgFp8, true, kTgEpiStore, 4, true>(d, st);
+    TileGemmArgs d{};
+    d.x = m.actq; d.xs = m.acts; d.x_rows = m.R; d.gather = nullptr;
+    d.w = w2; d.ws = s2; d.mtile_table = m.tiles; d.mtile_count = m.tile_count;
+    d.N = (int)m.H; d.K = (int)m.I; d.I = 0;
+    d.mtiles = m.max_tiles; d.ntiles = (int)((m.H + kTgBN - 1) / kTgBN);
+    d.out = m.y; d.out_dtype = m.dtype; d.bias = nullptr; d.bias_dtype = KQ_DTYPE_NONE;
+    if (m.nrb == 5) tg_launch<kTgFp8, true, kTgEpiStore, 5, true>(d, st);
+    else tg_launch<kTgFp8, true, kTgEpiStore, 4, true>(d, st);
+  }
 
   hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)m.tokens), dim3(256), 0, st, m.y, m.dtype, m.inv, topk_w,
                      m.top_k, (int)m.H, (uint16_t*)out);

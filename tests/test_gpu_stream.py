@@ -8,14 +8,15 @@ import numpy as np
 import pytest
 import torch
 
-from gpu_helpers import banner, bits, check_block_fp8, check_fp8, np32
+from gpu_helpers import assert_moe_close, banner, bits, check_block_fp8, check_fp8, np32
 from kairyu_amd.kernels import quant_gemm_hip as hip
-from kairyu_amd.moe import BlockFp8ExpertMlp
+from kairyu_amd.moe import BlockFp8ExpertMlp, GroupedBlockFp8Experts
 from kairyu_amd.quant.block_fp8 import quantize_block_fp8
 from kairyu_amd.quant.fp8 import quantize_fp8
 from kairyu_amd.quant.int8 import quantize_int8_weight
 from kairyu_amd.quant.linear import BlockFp8Linear, Fp8Linear, Int8Linear
 from oracle import linear as olinear
+from oracle import moe as omoe
 
 pytestmark = pytest.mark.gpu
 
@@ -124,3 +125,30 @@ def test_block_fp8_launch_quantizes_as_the_quantizer(cuda, dtype):
     finite = [0, 1, 2, 5, 6, 7]
     assert np.array_equal(bits(out)[finite], bits(want)[finite])
     assert torch.equal(torch.isnan(out), torch.isnan(want))
+
+
+# average rows per expert on both sides of each row tile's limit (2, 6 and 16
+# rows; then the tile engine), experts with none and with several tiles
+@pytest.mark.parametrize("tokens,experts,top_k", [(8, 16, 4), (9, 16, 4), (24, 16, 4), (25, 16, 4),
+                                                  (64, 16, 4), (65, 16, 4), (40, 128, 2)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_moe_row_tiles_match_oracle(cuda, tokens, experts, top_k, dtype):
+    hidden, inter = 384, 256
+    g = _gen(tokens * experts)
+    q13, s13 = quantize_block_fp8(torch.randn(experts, 2 * inter, hidden, generator=g) * 0.05)
+    q2, s2 = quantize_block_fp8(torch.randn(experts, hidden, inter, generator=g) * 0.05)
+    pack = GroupedBlockFp8Experts.from_tensors(*(t.to(cuda) for t in (q13, s13, q2, s2)))
+    x = torch.randn(tokens, hidden, generator=g).to(dtype)
+    logits = torch.randn(tokens, experts, generator=g)
+    logits[:, 0] += 3.0  # one expert holds nearly every token
+    logits[:, -1] -= 9.0
+    banner(f"moe row tiles tokens={tokens} E={experts} k={top_k} {dtype}")
+    out, idx, w = pack.forward_logits(x.to(cuda), logits.to(cuda), top_k)
+    name = str(dtype).split(".")[1]
+    want = omoe.moe_forward(np32(x), idx.cpu().numpy(), w.cpu().numpy(), bits(q13), s13.numpy(), bits(q2),
+                            s2.numpy(), name)
+    # the normwise bound of narrow layers (test_gpu_moe.py); a flipped e4m3
+    # activation moves an output by the same relative amount whatever its
+    # dtype, and 8 ulps of bf16 are 64 of fp16 (oracle.parity.moe_check)
+    assert_moe_close(np32(out), want, name, label=f"T={tokens} E={experts}", normwise=2e-2,
+                     ulps=8.0 if dtype == torch.bfloat16 else 64.0)
