@@ -186,9 +186,9 @@ static inline int moe_nrb(int64_t routed_rows, int64_t experts) {
 // flight per CU; the streaming kernel's cost grows with its row tile, so that
 // is the smallest that holds nearly every expert's rows at an even routing
 // (a further tile reads the expert's weights again).  C5's widths, whole call
-// (graph replay; before, after): 16 tokens (8-row tiles) 116 -> 84 us, 32
-// (8) 157 -> 102, 64 (16) 159 -> 137, 128 (32) 161 -> 139, 256 (32) 165 ->
-// 152; 512 tokens take 174 us with 256-row tiles and 250 with 64-row ones.
+// (graph replay; before, after): 16 tokens (8-row tiles) 116 -> 78 us, 32
+// (8) 157 -> 97, 64 (16) 159 -> 117, 128 (32) 161 -> 134, 256 (32) 165 ->
+// 143; 512 tokens take 174 us with 256-row tiles and 250 with 64-row ones.
 static inline int moe_stream_rows(int64_t routed_rows, int64_t experts) {
   if (routed_rows <= 2 * experts) return 8;
   if (routed_rows <= 6 * experts) return 16;
@@ -848,20 +848,21 @@ static MoeCall moe_call(const void* hidden, int dtype, int64_t tokens, int64_t H
 // Both expert projections with the weight-streaming kernel: gate_up stores
 // silu(gate) * up in the activation dtype, and down quantizes it itself (row
 // tiles of 8 or 16) or after the block quantizer.  Workgroups are small (an
-// expert's projection is many), 2 waves of 2 or 4 column tiles: more waves
-// leave each one or two K blocks of down's few (C5 at 16 tokens, 2 waves and 2
-// tiles 84 us, 4 waves 91, 4 tiles 92; at 64 tokens 4 tiles 137, 2 tiles 159).
+// expert's projection is many of them), with rings of two stages so that
+// several share a CU, and few waves, since down's K has few blocks: C5's call
+// at 16 / 64 / 128 tokens took 84 / 137 / 139 us with rings of three stages
+// and two waves, 78 / 117 / 134 as below; at 16 rows a tile, down with two
+// waves and four tiles takes 5 us more, gate_up with four tiles 10.
 static void moe_stream_gate_up(const MoeCall& m, const StreamArgs& a, hipStream_t st) {
   constexpr int DT = KQ_DTYPE_BF16;  // (of no use to quantized rows)
-  if (m.few == 8) sg_launch_form<kSgBlock, false, 1, 2, 2, 3, 1, true, DT>(a, m.max_tiles, st);
-  else if (m.few == 16) sg_launch_form<kSgBlock, false, 1, 4, 2, 2, 1, true, DT>(a, m.max_tiles, st);
-  else sg_launch_form<kSgBlock, false, 2, 2, 2, 3, 1, true, DT>(a, m.max_tiles, st);
+  if (m.few <= 16) sg_launch_form<kSgBlock, false, 1, 2, 4, 2, 1, true, DT>(a, m.max_tiles, st);
+  else sg_launch_form<kSgBlock, false, 2, 4, 3, 2, 1, true, DT>(a, m.max_tiles, st);
 }
 
 template <int DT>
 static void moe_stream_down_raw(const MoeCall& m, const StreamArgs& a, hipStream_t st) {
-  if (m.few == 8) sg_launch_form<kSgBlock, true, 1, 2, 2, 3, 1, false, DT>(a, m.max_tiles, st);
-  else sg_launch_form<kSgBlock, true, 1, 4, 2, 3, 2, false, DT>(a, m.max_tiles, st);
+  if (m.few == 8) sg_launch_form<kSgBlock, true, 1, 2, 2, 2, 1, false, DT>(a, m.max_tiles, st);
+  else sg_launch_form<kSgBlock, true, 1, 4, 3, 2, 2, false, DT>(a, m.max_tiles, st);
 }
 
 static void moe_stream_experts(const MoeCall& m, const uint8_t* w13, const float* s13, const uint8_t* w2,
@@ -889,7 +890,7 @@ static void moe_stream_experts(const MoeCall& m, const uint8_t* w13, const float
   }
   launch_act_quant_blocks(m.act, m.dtype, m.R, m.I, m.I, m.actq, m.acts, st);
   d.x = m.actq; d.x_bytes = (uint32_t)((int64_t)m.R * m.I); d.xs = m.acts; d.x_rows = m.R;
-  sg_launch_form<kSgBlock, false, 2, 2, 2, 3, 1, false, KQ_DTYPE_BF16>(d, m.max_tiles, st);
+  sg_launch_form<kSgBlock, false, 2, 4, 3, 2, 1, false, KQ_DTYPE_BF16>(d, m.max_tiles, st);
 }
 
 // After the chunk histograms and the token quantization: the stable sort's
