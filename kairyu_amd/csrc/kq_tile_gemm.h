@@ -154,27 +154,6 @@ KQ_DEV void tg_dma4(i32x4 rsrc, uint32_t lds, int32_t voff, int32_t soff) {
   kq_rbl_lds(rsrc, (tg_lds_ptr)(uintptr_t)lds, 4, voff, soff, 0, 0);
 }
 
-// Two values rounded (to nearest even) to the 16-bit dtype and packed, low
-// half first: one v_cvt_pk_bf16_f32 / v_cvt_pk_f16_f32.
-typedef __bf16 tg_bf16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 tg_f16x2 __attribute__((ext_vector_type(2)));
-typedef float tg_f32x2 __attribute__((ext_vector_type(2)));
-KQ_DEV uint32_t tg_pack2(float lo, float hi, int dtype) {
-  const tg_f32x2 v = {lo, hi};
-  if (dtype == KQ_DTYPE_BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, tg_bf16x2));
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, tg_f16x2));
-}
-// The two values of a packed pair, widened to fp32.
-KQ_DEV float tg_lo(uint32_t p, int dtype) {
-  if (dtype == KQ_DTYPE_BF16) return __uint_as_float(p << 16);
-  return (float)__builtin_bit_cast(_Float16, (uint16_t)p);
-}
-KQ_DEV float tg_hi(uint32_t p, int dtype) {
-  if (dtype == KQ_DTYPE_BF16) return __uint_as_float(p & 0xffff0000u);
-  return (float)__builtin_bit_cast(_Float16, (uint16_t)(p >> 16));
-}
-
-
 template <int FMT> struct TgTraits;
 template <> struct TgTraits<kTgFp8> { using Acc = f32x4; };
 template <> struct TgTraits<kTgI8> { using Acc = i32x4; };
@@ -595,13 +574,13 @@ tile_gemm_kernel(TileGemmArgs a) {
   #pragma unroll
             for (int h = 0; h < 2; ++h) {
               // the pair q = 2h, 2h + 1, each rounding a packed conversion
-              const uint32_t gp = tg_pack2(acc[j][mb][2 * h], acc[j][mb][2 * h + 1], ODT);
-              const uint32_t up = tg_pack2(acc[j + 4][mb][2 * h], acc[j + 4][mb][2 * h + 1], ODT);
-              const float g0 = tg_lo(gp, ODT), g1 = tg_hi(gp, ODT);
-              const uint32_t sp = tg_pack2(g0 * __builtin_amdgcn_rcpf(1.0f + __expf(-g0)),
+              const uint32_t gp = pack_act2(acc[j][mb][2 * h], acc[j][mb][2 * h + 1], ODT);
+              const uint32_t up = pack_act2(acc[j + 4][mb][2 * h], acc[j + 4][mb][2 * h + 1], ODT);
+              const float g0 = act_lo(gp, ODT), g1 = act_hi(gp, ODT);
+              const uint32_t sp = pack_act2(g0 * __builtin_amdgcn_rcpf(1.0f + __expf(-g0)),
                                            g1 * __builtin_amdgcn_rcpf(1.0f + __expf(-g1)), ODT);
-              const uint32_t vp = tg_pack2(tg_lo(sp, ODT) * tg_lo(up, ODT), tg_hi(sp, ODT) * tg_hi(up, ODT), ODT);
-              amax[mb] = fmaxf(amax[mb], fmaxf(fabsf(tg_lo(vp, ODT)), fabsf(tg_hi(vp, ODT))));
+              const uint32_t vp = pack_act2(act_lo(sp, ODT) * act_lo(up, ODT), act_hi(sp, ODT) * act_hi(up, ODT), ODT);
+              amax[mb] = fmaxf(amax[mb], fmaxf(fabsf(act_lo(vp, ODT)), fabsf(act_hi(vp, ODT))));
               pv[j][mb][h] = vp;
             }
           }
@@ -629,7 +608,7 @@ tile_gemm_kernel(TileGemmArgs a) {
             float v[4];
   #pragma unroll
             for (int q = 0; q < 4; ++q)
-              v[q] = fminf(fmaxf(div_by_recip((q & 1) ? tg_hi(pv[j][mb][q >> 1], ODT) : tg_lo(pv[j][mb][q >> 1], ODT), s, rs),
+              v[q] = fminf(fmaxf(div_by_recip((q & 1) ? act_hi(pv[j][mb][q >> 1], ODT) : act_lo(pv[j][mb][q >> 1], ODT), s, rs),
                                  -448.0f), 448.0f);
             const int col = 64 * wn + 16 * j + 4 * lg;
             *(uint32_t*)(stg + tg_stage_off4(lrow, col >> 2)) =
@@ -663,16 +642,14 @@ tile_gemm_kernel(TileGemmArgs a) {
           for (int mb = 0; mb < NRB; ++mb) {
             const int grow = row0 + trow(mb);
             const float xsc = eX[trow(mb)];
-            uint16_t o[4];
+            float g[4], u[4];
   #pragma unroll
             for (int q = 0; q < 4; ++q) {
-              const float g = __fadd_rn(__fmul_rn(__fmul_rn((float)acc[j][mb][q], xsc), wsg[q]), bg[q]);
-              const float u = __fadd_rn(__fmul_rn(__fmul_rn((float)acc[j + 4][mb][q], xsc), wsu[q]), bu[q]);
-              o[q] = swiglu_bits(g, u, ODT);
+              g[q] = __fadd_rn(__fmul_rn(__fmul_rn((float)acc[j][mb][q], xsc), wsg[q]), bg[q]);
+              u[q] = __fadd_rn(__fmul_rn(__fmul_rn((float)acc[j + 4][mb][q], xsc), wsu[q]), bu[q]);
             }
-            if (grow < row_end && col < I)
-              *(u32x2*)((uint16_t*)a.out + (int64_t)grow * I + col) =
-                  u32x2{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
+            const u32x2 o = u32x2{swiglu_bits2(g[0], u[0], g[1], u[1], ODT), swiglu_bits2(g[2], u[2], g[3], u[3], ODT)};
+            if (grow < row_end && col < I) *(u32x2*)((uint16_t*)a.out + (int64_t)grow * I + col) = o;
           }
         }
       } else if (ksplit > 1) {
@@ -739,7 +716,7 @@ tile_gemm_kernel(TileGemmArgs a) {
                   if (!BLOCK) v[q] = __fmul_rn(__fmul_rn(v[q], xsc), wsc[q]);
                   v[q] = __fadd_rn(v[q], bv[q]);
                 }
-                const u32x2 word = u32x2{tg_pack2(v[0], v[1], ODT), tg_pack2(v[2], v[3], ODT)};
+                const u32x2 word = u32x2{pack_act2(v[0], v[1], ODT), pack_act2(v[2], v[3], ODT)};
                 const uint16_t o[4] = {(uint16_t)word[0], (uint16_t)(word[0] >> 16), (uint16_t)word[1],
                                        (uint16_t)(word[1] >> 16)};
                 if (staged) {

@@ -1153,23 +1153,25 @@ w4a16_prefill_kernel(W4Args a, int mblocks, int tiles, int ksplit) {
       for (int i = 0; i < TM; ++i) {
         const int m = m0 + (wm * TM + i) * 16 + c;
         if (m >= a.M) continue;
-        uint16_t o[4];
+        float gv[4], uv[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          float gv = acc[2 * pp][i][q], uv = acc[2 * pp + 1][i][q];
+          gv[q] = acc[2 * pp][i][q];
+          uv[q] = acc[2 * pp + 1][i][q];
           if (a.bias_dtype != KQ_DTYPE_NONE) {
-            gv = __fadd_rn(gv, bg[q]);
-            uv = __fadd_rn(uv, bu[q]);
+            gv[q] = __fadd_rn(gv[q], bg[q]);
+            uv[q] = __fadd_rn(uv[q], bu[q]);
           }
-          o[q] = swiglu_bits(gv, uv, a.out_dtype);
         }
+        const uint32_t lo = swiglu_bits2(gv[0], uv[0], gv[1], uv[1], a.out_dtype);
+        const uint32_t hi = swiglu_bits2(gv[2], uv[2], gv[3], uv[3], a.out_dtype);
         uint16_t* dst = a.out + (int64_t)m * width + oc;
         if (oc + 3 < width) {
-          *(u32x2*)dst = u32x2{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
+          *(u32x2*)dst = u32x2{lo, hi};
         } else {
 #pragma unroll
           for (int q = 0; q < 4; ++q)
-            if (oc + q < width) dst[q] = o[q];
+            if (oc + q < width) dst[q] = (uint16_t)((q < 2 ? lo : hi) >> (16 * (q & 1)));
         }
       }
     }
@@ -1328,15 +1330,18 @@ swiglu_kernel(const uint16_t* __restrict__ src, int64_t ld_src, int interleaved,
   const int64_t idx = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 2;
   if (idx >= M * I) return;
   const int64_t m = idx / I, n = idx % I;  // I even: both outputs in row m
+  float g[2], u[2];
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     const int64_t c = n + e;
     const int64_t gc = interleaved ? (c >> 4) * 32 + (c & 15) : c;
     const int64_t uc = interleaved ? gc + 16 : I + c;
-    const float g = load_as_f32(src + m * ld_src, dtype, gc);
-    const float u = load_as_f32(src + m * ld_src, dtype, uc);
-    dst[m * I + c] = swiglu_bits(g, u, dtype);
+    g[e] = load_as_f32(src + m * ld_src, dtype, gc);
+    u[e] = load_as_f32(src + m * ld_src, dtype, uc);
   }
+  const uint32_t o = swiglu_bits2(g[0], u[0], g[1], u[1], dtype);
+  dst[m * I + n] = (uint16_t)o;
+  dst[m * I + n + 1] = (uint16_t)(o >> 16);
 }
 
 // AWQ word (k, c) holds column 8c + [0,2,4,6,1,3,5,7][i] in nibble i, so
