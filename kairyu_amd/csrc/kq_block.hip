@@ -4,8 +4,10 @@
 //
 //   * M <= 64: the weight-streaming kernel of kq_stream_gemm.h, HBM-bound; up
 //     to 16 rows it quantizes the activations itself.
-//   * M > 64: the persistent tile engine of kq_tile_gemm.h.
+//   * M <= 256: the panel kernel of kq_panel_gemm.h.
+//   * M > 256: the persistent tile engine of kq_tile_gemm.h.
 #include "kq_common.h"
+#include "kq_panel_gemm.h"
 #include "kq_stream_gemm.h"
 #include "kq_tile_gemm.h"
 
@@ -86,6 +88,12 @@ extern "C" int kq_block_fp8_gemm(const uint8_t* xq, const float* xs, const uint8
     StreamArgs a = block_stream_args(w, ws, bias, bias_dtype, out, out_dtype, m, n, k);
     block_quantized(a, xq, xs);
     sg_launch<kSgBlock, false>(a, (hipStream_t)stream);
+    return check_launch("kq_block_fp8_gemm");
+  }
+  if (m <= 256) {
+    StreamArgs a = block_stream_args(w, ws, bias, bias_dtype, out, out_dtype, m, n, k);
+    block_quantized(a, xq, xs);
+    pg_launch_block(a, (hipStream_t)stream);
     return check_launch("kq_block_fp8_gemm");
   }
   TileGemmArgs a{};

@@ -10,12 +10,15 @@
 //
 // Kernels:
 //   * M <= 64: the weight-streaming kernel of kq_stream_gemm.h.  HBM-bound.
+//   * M <= 256: the panel kernel of kq_panel_gemm.h where its panels fill the
+//     CUs (and 33 to 64 rows against many weight rows).
 //   * M > 64 with at least one 256x256 tile per CU: the persistent tile
 //     engine of kq_tile_gemm.h (LDS DMA double buffering, XCD-grouped tiles).
 //   * other M > 64: 128x128x128 workgroup tiles, 4 waves of 64x64, LDS
 //     double buffer with an XOR chunk swizzle (twice the workgroups of the
 //     256x256 engine for shapes that would leave CUs idle).
 #include "kq_common.h"
+#include "kq_panel_gemm.h"
 #include "kq_splitk.h"
 #include "kq_stream_gemm.h"
 #include "kq_tile_gemm.h"
@@ -226,8 +229,37 @@ static void launch_stream(const uint8_t* xq, const uint8_t* w, int K, const Epi&
   constexpr int SF = FMT == kFmtI8 ? kSgI8 : kSgFp8;
   StreamArgs a = stream_args(w, K, ep);
   a.x = xq; a.x_bytes = (uint32_t)((int64_t)ep.M * K); a.xs = ep.xscale;
+  if (ep.M > 32 && sg_form((ep.N + 15) / 16, K) == kSgMany) {
+    const PanelArgs p{a, 1, nullptr};
+    if (ep.swiglu) pg_launch_64<SF, true>(p, stream);
+    else pg_launch_64<SF, false>(p, stream);
+    return;
+  }
   if (ep.swiglu) sg_launch<SF, true>(a, stream);
   else sg_launch<SF, false>(a, stream);
+}
+
+// 65 to 256 rows: the panel kernel's form, nt = 0 where the tile engine or
+// the 128x128 kernel runs instead.
+static PanelForm panel_form(int64_t m, int64_t n, int64_t k) {
+  if (m <= 64 || m > 256 || k % 16 != 0 || k > 65536) return PanelForm{0, 0, 0, 1};
+  return pg_form(m, (n + 15) / 16, (int)((k + 127) / 128));
+}
+
+template <int FMT>
+static void launch_panel(const uint8_t* xq, const uint8_t* w, int K, const Epi& ep, PanelForm f,
+                         void* workspace, size_t ws_bytes, hipStream_t stream) {
+  constexpr int SF = FMT == kFmtI8 ? kSgI8 : kSgFp8;
+  if (!workspace || (size_t)f.splits * (size_t)ep.M * (size_t)ep.N * 4 > ws_bytes) f.splits = 1;
+  PanelArgs p{stream_args(w, K, ep), f.splits, (uint32_t*)workspace};
+  p.s.x = xq; p.s.x_bytes = (uint32_t)((int64_t)ep.M * K); p.s.xs = ep.xscale;
+  if (ep.swiglu) pg_launch<SF, true>(p, f, stream);
+  else pg_launch<SF, false>(p, f, stream);
+  if (f.splits > 1) {
+    ReduceArgs r{workspace, f.splits, ep.M, ep.N, ep.xscale, ep.wscale, ep.ws_per_channel,
+                 ep.bias, ep.bias_dtype, ep.out, ep.out_dtype, ep.acc_out, ep.swiglu};
+    launch_splitk_reduce(FMT == kFmtI8 ? kReduceI8 : kReduceFp8, r, stream);
+  }
 }
 
 // One fp16 / bf16 row, quantized in the launch.
@@ -284,9 +316,10 @@ static int run_w8a8(const char* what, const uint8_t* xq, const uint8_t* w, int64
   }
   if (m == 0) return KQ_OK;
   const int K = (int)k;
-  if (ep.swiglu && !(m <= 64 && K % 16 == 0 && ((uintptr_t)xq % 16) == 0 && ((uintptr_t)w % 16) == 0 &&
+  const PanelForm panel = panel_form(m, n, k);
+  if (ep.swiglu && !((m <= 64 || panel.nt) && K % 16 == 0 && ((uintptr_t)xq % 16) == 0 && ((uintptr_t)w % 16) == 0 &&
                      n * k < ((int64_t)1 << 31) && m * k < ((int64_t)1 << 31))) {
-    set_error("%s: the SwiGLU epilogue runs in the weight-streaming kernel only (m=%lld k=%lld)",
+    set_error("%s: the SwiGLU epilogue runs in the streaming and panel kernels only (m=%lld k=%lld)",
               what, (long long)m, (long long)k);
     return KQ_EINVAL;
   }
@@ -302,6 +335,8 @@ static int run_w8a8(const char* what, const uint8_t* xq, const uint8_t* w, int64
   }
   if (m <= 64 && m * k < ((int64_t)1 << 31) && k < ((int64_t)1 << 26)) {
     launch_stream<FMT>(xq, w, K, ep, stream);
+  } else if (panel.nt) {
+    launch_panel<FMT>(xq, w, K, ep, panel, workspace, ws_bytes, stream);
   }
   else if (const int splits = tile_engine_splits(m, n, K, workspace, ws_bytes)) {
     // persistent 256x256 MFMA tiles (kq_tile_gemm.h), scales in the epilogue;
@@ -395,7 +430,8 @@ extern "C" size_t kq_w8a8_workspace_size(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k <= 0 || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff) return 0;
   const size_t plane = (size_t)m * (size_t)n * 4;
   if (m <= 64) return 0;  // the weight-streaming kernel splits K within a workgroup only
-  const int s = tile_engine_splits(m, n, (int)k, (const void*)1, (size_t)-1);
+  const PanelForm panel = panel_form(m, n, k);
+  const int s = std::max(panel.nt ? panel.splits : 1, tile_engine_splits(m, n, (int)k, (const void*)1, (size_t)-1));
   return s > 1 ? plane * (size_t)s : 0;
 }
 
@@ -460,8 +496,8 @@ extern "C" int kq_w8a8_fp8_linear(const void* x, int x_dtype, int64_t ldx, const
 // CUs) run the tile engine with the SwiGLU store epilogue: each tile pairs
 // gate columns [n0, n0 + 128) with up columns [I + n0, I + n0 + 128), so the
 // [M, 2I] projection output never reaches memory.  Shapes of M <= 64 run the
-// weight-streaming kernel with the SwiGLU epilogue (each 16-row weight tile is
-// 8 gate rows and the matching 8 up rows).  Other shapes run the packed
+// weight-streaming kernel, up to 256 rows the panel kernel, with the SwiGLU
+// epilogue (each 16-row weight tile is 8 gate rows and the matching 8 up rows).  Other shapes run the packed
 // linear into the workspace and the elementwise pass.  All produce the bits
 // of the packed linear followed by kq_swiglu.
 static bool swiglu_fused_applies(int64_t m, int64_t i_width, int64_t k, const void* x, int64_t ldx,
@@ -484,8 +520,9 @@ static int run_swiglu_linear(const char* what, const void* x, int x_dtype, int64
   }
   const int64_t n = 2 * i_width;
   Epi ep{nullptr, wscale, ws_per_channel, bias, bias_dtype, out, x_dtype, nullptr, (int)m, (int)n};
+  const bool panel = panel_form(m, n, k).nt != 0;
   if (m > 0 && m <= 0x7fffffff && k >= 1 && k <= 65536 && ldx >= k && x != nullptr &&
-      (x_dtype == KQ_DTYPE_F16 || x_dtype == KQ_DTYPE_BF16) &&
+      (x_dtype == KQ_DTYPE_F16 || x_dtype == KQ_DTYPE_BF16) && !panel &&
       swiglu_fused_applies(m, i_width, k, x, ldx, w)) {
     const size_t xq_bytes = ((size_t)m * (size_t)k + 255) / 256 * 256;
     const size_t xs_bytes = ((size_t)m * 4 + 255) / 256 * 256;
@@ -513,9 +550,9 @@ static int run_swiglu_linear(const char* what, const void* x, int x_dtype, int64
     tg_launch<FMT == kFmtI8 ? kTgI8 : kTgFp8, false, kTgEpiSwiGluStore>(a, stream);
     return check_launch(what);
   }
-  if (m >= 1 && m <= 64 && k % 16 == 0 && k <= 65536 && ((uintptr_t)w % 16) == 0 &&
+  if (m >= 1 && (m <= 64 || panel) && k % 16 == 0 && k <= 65536 && ((uintptr_t)w % 16) == 0 &&
       ((uintptr_t)workspace % 16) == 0 && n * k < ((int64_t)1 << 31)) {
-    // few rows: the weight-streaming kernel (one-row fused quantization
+    // few rows: the streaming and panel kernels (one-row fused quantization
     // or the per-token quantizer first) with the SwiGLU epilogue
     ep.swiglu = 1;
     return run_linear<FMT>(what, x, x_dtype, ldx, scale_mode, scale_in, w, m, n, k, ep, workspace,

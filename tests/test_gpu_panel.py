@@ -1,0 +1,75 @@
+"""The panel GEMM (65 to 256 rows; from 33 with many weight rows) at the edges
+of its forms: one and two row tiles per wave, panels of 2 to 16 weight tiles,
+split K, K tails, ragged rows and columns, waves without rows."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_helpers import banner, bits, check_block_fp8, check_fp8, np32
+from kairyu_amd import _native
+from kairyu_amd.kernels import quant_gemm_hip as hip
+from kairyu_amd.quant.linear import BlockFp8Linear, Fp8Linear, Int8Linear
+from kairyu_amd.quant.packed import QuantLinearPack
+from oracle import linear as olinear
+from test_gpu_stream import _fill, _gen
+
+pytestmark = pytest.mark.gpu
+
+# (m, n, k): panels of 4 (unsplit, then split 3 ways), of 8 split 8 ways with a
+# tail, of 8 unsplit, of 12, of 16; one K block and a tail of 16 bytes
+SHAPES = [(65, 6200, 144), (130, 1004, 2832), (256, 1024, 8208), (96, 17000, 272), (129, 33000, 256),
+          (200, 50008, 128), (128, 8, 112), (40, 8600, 400), (64, 9000, 256)]
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_int8_panels_are_exact(cuda, m, n, k):
+    banner(f"panel int8 m={m} n={n} k={k}")
+    module = _fill(Int8Linear(k, n, True), _gen(n + k)).to(cuda)
+    x = torch.randn(m, k, generator=_gen(m)).to(torch.bfloat16)
+    acc = torch.empty(m, n, dtype=torch.int32, device=cuda)
+    out = hip.int8_linear_forward(x.to(cuda), module, accumulators=acc)
+    want, _, _, want_acc = olinear.int8_forward(
+        np32(x), module.weight.cpu().numpy(), module.weight_scale.cpu().numpy(), np32(module.bias))
+    assert np.array_equal(acc.cpu().numpy().astype(np.int64), want_acc)
+    assert np.array_equal(np32(out), want)
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_fp8_panels_match_oracle(cuda, m, n, k):
+    banner(f"panel fp8 m={m} n={n} k={k}")
+    module = _fill(Fp8Linear(k, n, True), _gen(n + k)).to(cuda)
+    x = torch.randn(m, k, generator=_gen(m)).to(torch.float16)
+    check_fp8(module(x.to(cuda)), x, module, label=f"m={m} n={n} k={k}")
+
+
+@pytest.mark.parametrize("m", [65, 128, 129, 256])
+@pytest.mark.parametrize("n,k", [(200, 384), (5000, 256), (17000, 128), (72, 16384)])
+def test_block_fp8_panels_match_oracle(cuda, m, n, k):
+    banner(f"panel block fp8 m={m} n={n} k={k}")
+    module = _fill(BlockFp8Linear(k, n, True), _gen(n + k)).to(cuda)
+    x = torch.randn(m, k, generator=_gen(m)).to(torch.bfloat16)
+    check_block_fp8(module(x.to(cuda)), x, module, label=f"m={m} n={n} k={k}")
+
+
+# unsplit and split panels (the reduce pairs the columns), every panel width,
+# widths of odd eighths, rows of one and two row tiles per wave
+@pytest.mark.parametrize("kind,m,width,k,dtype", [
+    ("fp8", 65, 1000, 1024, torch.bfloat16), ("fp8", 200, 520, 8320, torch.float16),
+    ("fp8", 130, 9000, 272, torch.bfloat16), ("int8", 256, 17000, 256, torch.float16),
+    ("int8", 100, 26000, 144, torch.bfloat16), ("fp8", 50, 5004, 400, torch.bfloat16),
+    ("int8", 64, 4600, 512, torch.float16), ("int8", 129, 1004, 2048, torch.float16)])
+def test_swiglu_panels_give_the_two_pass_bits(cuda, kind, m, width, k, dtype):
+    banner(f"panel swiglu {kind} m={m} I={width} k={k}")
+    make = Fp8Linear if kind == "fp8" else Int8Linear
+    g = _gen(width)
+    pack = QuantLinearPack.create([_fill(make(k, width, True), g).to(cuda) for _ in range(2)])
+    x = torch.randn(m, k, generator=g).to(dtype).to(cuda)
+    fused = pack.swiglu(x)
+    packed = torch.cat(pack(x), dim=-1).contiguous()
+    two = torch.empty(m, width, device=cuda, dtype=dtype)
+    _native.call("kq_swiglu", packed.data_ptr(), packed.stride(0), 0, _native.dtype_code(dtype), two.data_ptr(),
+                 m, width, _native.stream_handle(cuda))
+    assert np.array_equal(bits(fused), bits(two))
