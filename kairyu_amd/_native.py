@@ -104,6 +104,8 @@ _load_error: str | None = None
 
 def _load() -> ctypes.CDLL:
     global _lib, _load_error
+    if _lib is not None:  # bound last, once every signature is set
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib

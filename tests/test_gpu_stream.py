@@ -152,3 +152,18 @@ def test_moe_row_tiles_match_oracle(cuda, tokens, experts, top_k, dtype):
     # dtype, and 8 ulps of bf16 are 64 of fp16 (oracle.parity.moe_check)
     assert_moe_close(np32(out), want, name, label=f"T={tokens} E={experts}", normwise=2e-2,
                      ulps=8.0 if dtype == torch.bfloat16 else 64.0)
+
+
+def test_one_row_of_any_pitch_gives_the_contiguous_rows_bits(cuda):
+    """One row counts as contiguous at any pitch; the kernels take one of at
+    least K."""
+    k, n = 256, 64
+    module = _fill(Fp8Linear(k, n, True), _gen(1)).to(cuda)
+    x = torch.randn(1, k, generator=_gen(2)).to(torch.bfloat16).to(cuda)
+    want = module(x)
+    banner("one-row pitches")
+    narrow = x.reshape(k, 1).t()
+    wide = torch.cat([x, x], dim=1)[:, :k]
+    assert narrow.is_contiguous() and narrow.stride(0) == 1 and wide.stride(0) == 2 * k
+    for row in (narrow, wide, x[0], x[None]):
+        assert np.array_equal(bits(module(row)).reshape(-1), bits(want).reshape(-1))
