@@ -326,7 +326,7 @@ int kq_block_fp8_linear(const void* x, int x_dtype, int64_t ldx, const uint8_t* 
 size_t kq_block_fp8_workspace_size(int64_t m, int64_t k);
 
 /* out [m, i_width] = silu(gate) * up of two block-FP8 projections [i_width, k]
- * of the same x, m <= 64, with the roundings of the two linears followed by
+ * of the same x, m <= 128, with the roundings of the two linears followed by
  * torch's silu and product (each projection's bias may be null, both of
  * bias_dtype).  Replaces act_fn(gate(x)) * up(x) of the expert MLP
  * (kairyu/models/moe.py:27-83). */

@@ -4,7 +4,12 @@
 //
 //   * M <= 64: the weight-streaming kernel of kq_stream_gemm.h, HBM-bound; up
 //     to 16 rows it quantizes the activations itself.
-//   * M <= 256: the panel kernel of kq_panel_gemm.h.
+//   * M <= 256: the panel kernel of kq_panel_gemm.h.  A SwiGLU launch goes up to
+//     128 rows: a layer's projections at 65 / 128 rows, two projections and
+//     elementwise passes before -> now, 4096 / 12288 203.3 -> 194.9 us / 237.7 ->
+//     227.3, 5120 / 6912 (a shard) 186.4 -> 168.6 / 224.1 -> 197.3; at 200 rows
+//     4096 / 12288 lost 2% (276.4 -> 281.0), its two row tiles reading the
+//     activations once per 64 columns and not once per 128.
 //   * M > 256: the persistent tile engine of kq_tile_gemm.h.
 #include "kq_common.h"
 #include "kq_panel_gemm.h"
@@ -54,6 +59,16 @@ static void block_raw(StreamArgs& a, const void* x, int64_t ldx) {
   a.x = x; a.ldx = (int)ldx; a.x_bytes = (uint32_t)(((int64_t)(a.M - 1) * ldx + a.K) * 2);
 }
 
+// Quantized rows: the streaming kernel up to 64 rows, the panel kernel up to
+// 256.  (Panels of 4 tiles from 33 rows up against many weight tiles, which
+// INT8 and FP8 take, gain nothing here: a layer of 4096 / 12288 at 33 / 48 / 64
+// rows 103.2 / 114.4 / 130.7 us streamed, 104.7 / 114.9 / 129.7 in panels.)
+template <bool SW>
+static void block_launch(const StreamArgs& a, hipStream_t st) {
+  if (a.M > 64) pg_launch_block<SW>(a, st);
+  else sg_launch<kSgBlock, SW>(a, st);
+}
+
 // e4m3 rows, then their block scales, in the workspace
 static size_t block_xq_bytes(int64_t m, int64_t k) { return ((size_t)m * (size_t)k + 255) / 256 * 256; }
 static size_t block_quant_bytes(int64_t m, int64_t k) {
@@ -84,16 +99,10 @@ extern "C" int kq_block_fp8_gemm(const uint8_t* xq, const float* xs, const uint8
   }
   const int bad = block_check_shape("kq_block_fp8_gemm", m, n, k);
   if (bad != KQ_OK || m == 0) return bad;
-  if (m <= 64) {
-    StreamArgs a = block_stream_args(w, ws, bias, bias_dtype, out, out_dtype, m, n, k);
-    block_quantized(a, xq, xs);
-    sg_launch<kSgBlock, false>(a, (hipStream_t)stream);
-    return check_launch("kq_block_fp8_gemm");
-  }
   if (m <= 256) {
     StreamArgs a = block_stream_args(w, ws, bias, bias_dtype, out, out_dtype, m, n, k);
     block_quantized(a, xq, xs);
-    pg_launch_block(a, (hipStream_t)stream);
+    block_launch<false>(a, (hipStream_t)stream);
     return check_launch("kq_block_fp8_gemm");
   }
   TileGemmArgs a{};
@@ -148,8 +157,8 @@ extern "C" int kq_block_fp8_swiglu_linear(const void* x, int x_dtype, int64_t ld
   }
   const int bad = block_check_shape("kq_block_fp8_swiglu_linear", m, i_width, k);
   if (bad != KQ_OK || m == 0) return bad;
-  if (m > 64 || ldx < k) {
-    set_error("kq_block_fp8_swiglu_linear: at most 64 rows of pitch >= k (m=%lld ldx=%lld)", (long long)m,
+  if (m > 128 || ldx < k) {
+    set_error("kq_block_fp8_swiglu_linear: at most 128 rows of pitch >= k (m=%lld ldx=%lld)", (long long)m,
               (long long)ldx);
     return KQ_EINVAL;
   }
@@ -164,6 +173,6 @@ extern "C" int kq_block_fp8_swiglu_linear(const void* x, int x_dtype, int64_t ld
   const int rc = block_quantize("kq_block_fp8_swiglu_linear", x, x_dtype, ldx, m, k, workspace, workspace_bytes, st);
   if (rc != KQ_OK) return rc;
   block_quantized(a, (const uint8_t*)workspace, (const float*)((uint8_t*)workspace + block_xq_bytes(m, k)));
-  sg_launch<kSgBlock, true>(a, st);
+  block_launch<true>(a, st);
   return check_launch("kq_block_fp8_swiglu_linear");
 }

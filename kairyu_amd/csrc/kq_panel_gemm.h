@@ -337,14 +337,19 @@ static void pg_launch(const PanelArgs& a, const PanelForm& f, hipStream_t stream
 // Block FP8, 65 to 256 rows (no split K): panels of 8, 4 or 2 tiles against
 // 128 rows, the widest that gives half the CUs a workgroup.  M = 200, us:
 // N = K = 4096 19.0 with 2 tiles, 24.7 with 4 (the tile engine 51); 24576 rows
-// K = 4096 63.9 with 8.
+// K = 4096 63.9 with 8.  Every form adds an element's K blocks in one order, so
+// a SwiGLU launch gives the bits of its two projections.
+template <bool SW>
 static inline void pg_launch_block(const StreamArgs& s, hipStream_t stream) {
   const PanelArgs a{s, 1, nullptr};
   const int64_t need = tg_device_cus() / 2, row_tiles = (s.M + 127) / 128;
-  auto units = [&](int nt) { return (s.N + 16 * nt - 1) / (16 * nt) * row_tiles; };
-  if (units(8) >= need) pg_launch_form<kSgBlock, 2, 4, 8, 3, false>(a, stream);
-  else if (units(4) >= need) pg_launch_form<kSgBlock, 2, 4, 4, 4, false>(a, stream);
-  else pg_launch_form<kSgBlock, 2, 4, 2, 4, false>(a, stream);
+  auto units = [&](int nt) {
+    const int cols = (SW ? 8 : 16) * nt;
+    return (s.N + cols - 1) / cols * row_tiles;
+  };
+  if (units(8) >= need) pg_launch_form<kSgBlock, 2, 4, 8, 3, SW>(a, stream);
+  else if (units(4) >= need) pg_launch_form<kSgBlock, 2, 4, 4, 4, SW>(a, stream);
+  else pg_launch_form<kSgBlock, 2, 4, 2, 4, SW>(a, stream);
 }
 
 // 33 to 64 rows against many weight tiles: panels of 4 tiles, several

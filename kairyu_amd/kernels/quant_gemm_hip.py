@@ -527,7 +527,7 @@ def _block_fp8_workspace(device: torch.device, m: int, k: int) -> torch.Tensor:
     return _workspace(device, need)
 
 
-BLOCK_SWIGLU_ROWS = 64
+BLOCK_SWIGLU_ROWS = 128
 
 
 def block_fp8_swiglu_forward(x: torch.Tensor, gate, up) -> torch.Tensor:

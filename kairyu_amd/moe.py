@@ -140,8 +140,8 @@ class BlockFp8ExpertMlp(nn.Module):
         return self.down_proj(nn.functional.silu(self.gate_proj(hidden)) * self.up_proj(hidden))
 
     def _fused_swiglu(self, hidden: torch.Tensor) -> bool:
-        """Whether gate, up and their SwiGLU run as one launch: a decode batch
-        through two plain block-FP8 projections (no hooks, no other forward
+        """Whether gate, up and their SwiGLU run as one launch: a batch of few
+        rows through two plain block-FP8 projections (no hooks, no other forward
         bound) of equal widths and alike biases."""
 
         from kairyu_amd.kernels import quant_gemm_hip as hip

@@ -11,6 +11,7 @@ import torch
 from gpu_helpers import banner, bits, check_block_fp8, check_fp8, np32
 from kairyu_amd import _native
 from kairyu_amd.kernels import quant_gemm_hip as hip
+from kairyu_amd.moe import BlockFp8ExpertMlp
 from kairyu_amd.quant.linear import BlockFp8Linear, Fp8Linear, Int8Linear
 from kairyu_amd.quant.packed import QuantLinearPack
 from oracle import linear as olinear
@@ -73,3 +74,26 @@ def test_swiglu_panels_give_the_two_pass_bits(cuda, kind, m, width, k, dtype):
     _native.call("kq_swiglu", packed.data_ptr(), packed.stride(0), 0, _native.dtype_code(dtype), two.data_ptr(),
                  m, width, _native.stream_handle(cuda))
     assert np.array_equal(bits(fused), bits(two))
+
+
+# panels of 2, 4 and 8 tiles (16, 32 and 64 columns), ragged rows and columns,
+# the first and last row counts of the launch and the two-pass form past them
+@pytest.mark.parametrize("m", [65, 100, 128, 129])
+@pytest.mark.parametrize("width,k,bias,dtype", [
+    (200, 384, True, torch.bfloat16), (4100, 256, False, torch.float16),
+    (8200, 128, True, torch.bfloat16), (72, 16384, False, torch.bfloat16)])
+def test_block_fp8_swiglu_panels_give_the_two_pass_bits(cuda, m, width, k, bias, dtype):
+    """Each form adds an element's K blocks in one order: the projections'
+    outputs through the elementwise pass, bit for bit."""
+    banner(f"panel block swiglu m={m} I={width} k={k}")
+    mlp = BlockFp8ExpertMlp(128, 128)
+    g = _gen(width)
+    mlp.gate_proj, mlp.up_proj = (_fill(BlockFp8Linear(k, width, bias), g) for _ in range(2))
+    mlp.down_proj = torch.nn.Identity()
+    mlp = mlp.to(cuda)
+    x = torch.randn(m, k, generator=g).to(dtype).to(cuda)
+    packed = torch.cat([mlp.gate_proj(x), mlp.up_proj(x)], dim=-1).contiguous()
+    two = torch.empty(m, width, device=cuda, dtype=dtype)
+    _native.call("kq_swiglu", packed.data_ptr(), packed.stride(0), 0, _native.dtype_code(dtype), two.data_ptr(),
+                 m, width, _native.stream_handle(cuda))
+    assert np.array_equal(bits(mlp(x)), bits(two))

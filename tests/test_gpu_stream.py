@@ -80,7 +80,7 @@ def test_block_fp8_rows_match_oracle(cuda, n, k, dtype):
 @pytest.mark.parametrize("n,k", [(200, 384), (5000, 256)])
 @pytest.mark.parametrize("bias", [False, True])
 def test_block_fp8_mlp_matches_its_projections(cuda, m, n, k, bias):
-    """The expert MLP, whose gate, up and SwiGLU are one launch up to 64 rows,
+    """The expert MLP, whose gate, up and SwiGLU are one launch,
     against down(silu(gate(x)) * up(x)) of the same modules: the sums of a
     gate or up column may be added in another order, so a rounding of the
     activation dtype apart (2^-8 relative in bf16, from both factors)."""
@@ -95,7 +95,7 @@ def test_block_fp8_mlp_matches_its_projections(cuda, m, n, k, bias):
     gate, up = mlp.gate_proj(x), mlp.up_proj(x)
     want = torch.nn.functional.silu(gate) * up
     torch.testing.assert_close(out.float(), want.float(), rtol=2.0 ** -6, atol=2.0 ** -9 * float(up.abs().max()))
-    if m == 65:  # past the launch's rows: the projections themselves
+    if m == 65:  # the panel kernel: the projections' order
         assert np.array_equal(bits(out), bits(want))
 
 
