@@ -512,7 +512,7 @@ def block_fp8_linear_forward(x: torch.Tensor, module, *, add_bias: bool = True) 
         raise ValueError(f"block FP8 kernel needs in_features % 128 == 0, got {k}")
     bias = _bias(module, add_bias)
     scale_inv = _f32(module.weight_scale_inv)
-    ws = _block_fp8_workspace(x.device, m, k)
+    ws = _block_fp8_scratch(x.device, m, k)
     _native.call(
         "kq_block_fp8_linear", flat.data_ptr(), _native.dtype_code(flat.dtype), flat.stride(0),
         module.weight.data_ptr(), scale_inv.data_ptr(), _native.ptr(bias),
@@ -522,9 +522,14 @@ def block_fp8_linear_forward(x: torch.Tensor, module, *, add_bias: bool = True) 
     return out if x.dim() == 2 else out.reshape(*x.shape[:-1], module.out_features)
 
 
-def _block_fp8_workspace(device: torch.device, m: int, k: int) -> torch.Tensor:
+def _block_fp8_scratch(device: torch.device, m: int, k: int) -> torch.Tensor:
+    """Room for a block-FP8 call's quantized rows and their scales, of the
+    call's own: torch's allocator keeps it to the calling stream, so calls on
+    several streams or threads never meet (the shared ``workspace`` buffer
+    holds for callers on one stream)."""
+
     need = _workspace_bytes("kq_block_fp8_workspace_size", _device_index(device), m, k)
-    return _workspace(device, need)
+    return torch.empty(need, device=device, dtype=torch.uint8)
 
 
 BLOCK_SWIGLU_ROWS = 128
@@ -542,7 +547,7 @@ def block_fp8_swiglu_forward(x: torch.Tensor, gate, up) -> torch.Tensor:
     bias = _bias(gate, gate._add_local_bias())
     bias_up = _bias(up, up._add_local_bias())
     scales, scales_up = _f32(gate.weight_scale_inv), _f32(up.weight_scale_inv)
-    ws = _block_fp8_workspace(x.device, m, k)
+    ws = _block_fp8_scratch(x.device, m, k)
     _native.call(
         "kq_block_fp8_swiglu_linear", flat.data_ptr(), _native.dtype_code(flat.dtype), flat.stride(0),
         gate.weight.data_ptr(), scales.data_ptr(), up.weight.data_ptr(), scales_up.data_ptr(),

@@ -167,3 +167,29 @@ def test_one_row_of_any_pitch_gives_the_contiguous_rows_bits(cuda):
     assert narrow.is_contiguous() and narrow.stride(0) == 1 and wide.stride(0) == 2 * k
     for row in (narrow, wide, x[0], x[None]):
         assert np.array_equal(bits(module(row)).reshape(-1), bits(want).reshape(-1))
+
+
+def test_block_fp8_calls_on_two_streams_do_not_meet(cuda):
+    """32 rows are quantized into scratch before the GEMM: calls queued on two
+    streams, a linear and an MLP's fused gate and up, each give the bits that
+    they give alone."""
+    n = k = 1024
+    module = _fill(BlockFp8Linear(k, n, False), _gen(1)).to(cuda)
+    mlp = BlockFp8ExpertMlp(128, 128)
+    mlp.gate_proj, mlp.up_proj = (_fill(BlockFp8Linear(k, n, False), _gen(s)) for s in (2, 3))
+    mlp.down_proj = torch.nn.Identity()
+    mlp = mlp.to(cuda)
+    calls = [module, mlp, module]
+    xs = [torch.randn(32, k, generator=_gen(10 + i)).to(torch.bfloat16).to(cuda) for i in range(6)]
+    want = [[f(x) for f in calls] for x in xs]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    banner("block fp8 on two streams")
+    got = [[] for _ in xs]
+    for _ in range(10):
+        for i, x in enumerate(xs):
+            with torch.cuda.stream(streams[i % 2]):
+                got[i] = [f(x) for f in calls]
+    torch.cuda.synchronize()
+    for a, b in zip(got, want):
+        assert all(np.array_equal(bits(p), bits(q)) for p, q in zip(a, b))

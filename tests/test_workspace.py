@@ -54,3 +54,45 @@ def test_devices_are_independent():
     pool, _ = _pool()
     a, b = pool.get(0, 64), pool.get(1, 128)
     assert a is not b and pool.get(0, 1) is a and pool.get(1, 1) is b
+
+
+def test_block_fp8_calls_have_scratch_of_their_own(monkeypatch):
+    """Block-FP8 linears take the room for their quantized rows from torch's
+    allocator, per call: two calls whose scratch is alive at once (two streams,
+    two threads) share no byte, and none of the device's shared buffer."""
+
+    from types import SimpleNamespace
+
+    from kairyu_amd import _native
+    from kairyu_amd.kernels import quant_gemm_hip as hip
+
+    spans, shared = [], torch.empty(1 << 16, dtype=torch.uint8)
+    alive = []
+
+    def call(name, *args):
+        at, nbytes = args[-3], args[-2]
+        assert nbytes >= 32 * 256 + 32 * 2 * 4
+        spans.append((at, at + nbytes))
+
+    empty = torch.empty
+
+    def keep(*args, **kwargs):
+        alive.append(empty(*args, **kwargs))
+        return alive[-1]
+
+    monkeypatch.setattr(_native, "call", call)
+    monkeypatch.setattr(_native, "workspace", lambda device, nbytes=0: shared)
+    monkeypatch.setattr(_native, "stream_handle", lambda device: 0)
+    monkeypatch.setattr(hip, "_device_index", lambda device: 0)
+    monkeypatch.setattr(hip, "_workspace_bytes", lambda entry, index, m, k: m * k + m * k // 32)
+    monkeypatch.setattr(hip, "_prepare", lambda x, module, scheme, **kw: (x, empty(32, 64, dtype=x.dtype)))
+    monkeypatch.setattr(torch, "empty", keep)
+    module = SimpleNamespace(weight=empty(64, 256, dtype=torch.uint8), weight_scale_inv=empty(1, 2), bias=None,
+                             in_features=256, out_features=64, _add_local_bias=lambda: True)
+    x = empty(32, 256, dtype=torch.bfloat16)
+    hip.block_fp8_linear_forward(x, module)
+    hip.block_fp8_linear_forward(x, module)
+    hip.block_fp8_swiglu_forward(x, module, module)
+    spans.append((shared.data_ptr(), shared.data_ptr() + shared.numel()))
+    spans.sort()
+    assert len(spans) == 4 and all(a[1] <= b[0] for a, b in zip(spans, spans[1:]))
