@@ -141,13 +141,15 @@ class BlockFp8ExpertMlp(nn.Module):
 
     def _fused_swiglu(self, hidden: torch.Tensor) -> bool:
         """Whether gate, up and their SwiGLU run as one launch: a batch of few
-        rows through two plain block-FP8 projections (no hooks, no other forward
-        bound) of equal widths and alike biases."""
+        rows through two plain block-FP8 projections (no hooks of their own or of
+        every module, no other forward bound) of equal widths and alike biases."""
 
         from kairyu_amd.kernels import quant_gemm_hip as hip
 
         gate, up = self.gate_proj, self.up_proj
         if not 0 < hidden.numel() <= hip.BLOCK_SWIGLU_ROWS * hidden.shape[-1]:
+            return False
+        if torch.nn.modules.module._has_any_global_hook():  # due on each projection's call
             return False
         for m in (gate, up):
             if type(m) is not BlockFp8Linear or not _plain(m):
