@@ -133,7 +133,8 @@ class BlockFp8ExpertMlp(nn.Module):
                                      shard_dim=1, **common)
 
     def forward(self, hidden: torch.Tensor) -> torch.Tensor:
-        if hidden.is_cuda and self._fused_swiglu(hidden):
+        # (a symbolic tracer's value is no tensor: it records the three projections)
+        if isinstance(hidden, torch.Tensor) and hidden.is_cuda and self._fused_swiglu(hidden):
             from kairyu_amd.kernels import quant_gemm_hip as hip
 
             return self.down_proj(hip.block_fp8_swiglu_forward(hidden, self.gate_proj, self.up_proj))
