@@ -11,10 +11,10 @@ from kairyu_amd.moe import BlockFp8ExpertMlp
 def test_hooks_keep_the_projections_calls():
     mlp, x = BlockFp8ExpertMlp(256, 128), torch.zeros(4, 256, dtype=torch.bfloat16)
     assert mlp._fused_swiglu(x)
-    for handle in (mlp.gate_proj.register_forward_hook(lambda *args: None),
-                   mlp.up_proj.register_forward_pre_hook(lambda *args: None),
-                   torch.nn.modules.module.register_module_forward_hook(lambda *args: None),
-                   torch.nn.modules.module.register_module_forward_pre_hook(lambda *args: None)):
+    every = torch.nn.modules.module
+    for register in (mlp.gate_proj.register_forward_hook, mlp.up_proj.register_forward_pre_hook,
+                     every.register_module_forward_hook, every.register_module_forward_pre_hook):
+        handle = register(lambda *args: None)
         assert not mlp._fused_swiglu(x)
         handle.remove()
         assert mlp._fused_swiglu(x)
