@@ -403,7 +403,9 @@ __global__ void __launch_bounds__(64 * NW) stream_gemm_kernel(StreamArgs a) {
     const uint8_t* xf = q + L::W;
     if constexpr (RAW && !BLOCK) {
       uint8_t* frag = mine + L::Frag;
-      *(uint16_t*)(frag + lane * 2) = sg_quant2<FMT, DT>(*(const uint32_t*)(xf + lane * 4), row_s, row_rs, row_ok);
+      const uint16_t q2 = sg_quant2<FMT, DT>(*(const uint32_t*)(xf + lane * 4), row_s, row_rs, row_ok);
+      // zeros past K whatever the scale: 0 / 0 under a given scale of zero is NaN
+      *(uint16_t*)(frag + lane * 2) = (wave + i * NW) * 128 + lane * 2 < K ? q2 : (uint16_t)0;
       xf = frag;
     } else if constexpr (RAW) {
       uint8_t* frag = mine + L::Frag;

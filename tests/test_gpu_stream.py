@@ -193,3 +193,17 @@ def test_block_fp8_calls_on_two_streams_do_not_meet(cuda):
     torch.cuda.synchronize()
     for a, b in zip(got, want):
         assert all(np.array_equal(bits(p), bits(q)) for p, q in zip(a, b))
+
+
+@pytest.mark.parametrize("k", [112, 144, 256])
+def test_a_static_scale_of_zero_gives_one_row_the_bits_of_two(cuda, k):
+    """One row is quantized in the launch: past K (112 and 144 end inside a
+    block of 128) it holds zeros, also where a scale of zero makes every
+    quotient infinite (clamped to 448) or, of a zero, NaN."""
+    module = _fill(Fp8Linear(k, 40, True, activation_dynamic=False), _gen(k)).to(cuda)
+    module.input_scale.zero_()
+    x = torch.randn(1, k, generator=_gen(3)).to(torch.bfloat16).to(cuda)
+    banner(f"static scale zero k={k}")
+    out = module(x)
+    assert torch.isfinite(out).all()
+    assert np.array_equal(bits(out), bits(module(x.expand(2, k).contiguous())[:1]))
