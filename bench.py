@@ -210,7 +210,8 @@ def gemm_launcher(workload, copies: int):
                          _native.stream_handle(device))
 
         nbytes = k * n // 2 + groups * (n // 8) * 4 + groups * n * 2 + m * k * 2 + m * n * 2
-        kernel = ("w4a16_gemv_kernel (M <= 16 decode GEMV)" if m <= 16
+        streamed = m > 16 and _native.w4a16_route(x16.dtype, False, m, n, k, group).kernel == "stream"
+        kernel = ("w4a16_gemv_kernel (M <= 16 decode GEMV)" if m <= 16 else "w4a16_stream_kernel" if streamed
                   else "w4a16_prefill_kernel (+ its fp16 staging pass)")
         return launch, nbytes, 2 * m * n * k, kernel
     fp8 = isinstance(module, Fp8Linear)
@@ -234,12 +235,11 @@ def gemm_launcher(workload, copies: int):
                          _native.stream_handle(device))
 
     nbytes = n * k + 4 * n + m * k + 4 * m + 2 * m * n
-    # the launcher's dispatch in kq_w8a8.hip: the weight-streaming kernel up
-    # to M = 64, tile engine above
-    if m <= 64:
-        kernel = "stream_gemm_kernel"
-    else:
-        kernel = "tile_gemm_kernel (+ split-K reduce when used)"
+    route = _native.w8a8_route(m, n, k)
+    kernel = {"generic": "w8a8_generic_kernel", "stream": "stream_gemm_kernel", "panel": "panel_gemm_kernel",
+              "tile": "tile_gemm_kernel", "square": "w8a8_tile_kernel"}[route.kernel]
+    if route.splits > 1:
+        kernel += " + split-K reduce"
     return launch, nbytes, 2 * m * n * k, kernel
 
 

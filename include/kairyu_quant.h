@@ -43,6 +43,13 @@ extern "C" {
 #define KQ_DTYPE_BF16 1
 #define KQ_DTYPE_F32 2
 
+/* Kernels of a GEMM, as the *_route entries name them. */
+#define KQ_ROUTE_GENERIC 0 /* one thread per output; W4A16: the decode GEMV or the skinny kernel */
+#define KQ_ROUTE_STREAM 1  /* weight-streaming kernel                     */
+#define KQ_ROUTE_PANEL 2   /* panel kernel                                */
+#define KQ_ROUTE_TILE 3    /* tile engine; W4A16: prefill kernel          */
+#define KQ_ROUTE_SQUARE 4  /* 128 x 128 tiles                             */
+
 /* Library version (major*10000 + minor*100 + patch). */
 int kq_version(void);
 
@@ -145,6 +152,19 @@ size_t kq_w8a8_swiglu_workspace_size(int64_t m, int64_t i_width, int64_t k);
  * the reference (its GPU path calls torch._scaled_mm / Triton, which allocate
  * through torch). */
 size_t kq_w8a8_workspace_size(int64_t m, int64_t n, int64_t k);
+
+/* The kernel that a GEMM of this shape runs, with 16-byte aligned operands and
+ * the workspace of its size entry, for labels and tests (host only, nothing is
+ * launched): route[0] a KQ_ROUTE_* value, route[1] 16-row weight tiles of a
+ * workgroup, route[2] its waves (both 0 for KQ_ROUTE_GENERIC and W4A16's
+ * prefill kernel), route[3] K splits over workgroups.  swiglu: n = 2 * i_width
+ * for W8A8 and W4A16, i_width for block FP8 (at most 128 rows).  W4A16: the
+ * tiled operand, gathered through an act-order permutation or not.  No
+ * counterpart in the reference. */
+int kq_w8a8_route(int64_t m, int64_t n, int64_t k, int swiglu, int32_t* route);
+int kq_block_fp8_route(int64_t m, int64_t n, int64_t k, int swiglu, int32_t* route);
+int kq_w4a16_route(int x_dtype, int gathered, int64_t m, int64_t n, int64_t k, int group_size,
+                   int swiglu, int32_t* route);
 
 /* AWQ W4A16 ("gemm" layout): qweight int32 [k, n/8] packed along n in order
  * [0,2,4,6,1,3,5,7], qzeros int32 [k/g, n/8] same packing, scales fp16 [k/g, n].

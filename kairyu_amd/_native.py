@@ -13,6 +13,7 @@ import ctypes
 import os
 import threading
 from pathlib import Path
+from typing import NamedTuple
 
 import torch
 
@@ -86,6 +87,9 @@ _SIGNATURES: dict[str, list] = {
     "kq_block_fp8_swiglu_linear": [
         _P, _I, _I64, _P, _P, _P, _P, _P, _P, _I, _P, _I64, _I64, _I64, _P, _SZ, _P,
     ],
+    "kq_w8a8_route": [_I64, _I64, _I64, _I, _P],
+    "kq_block_fp8_route": [_I64, _I64, _I64, _I, _P],
+    "kq_w4a16_route": [_I, _I, _I64, _I64, _I64, _I, _I, _P],
     "kq_moe_workspace_size": [_I64, _I64, _I64, _I64, _I],
     "kq_peak_stream_read": [_P, _I64, _I, _P, _P],
     "kq_peak_mfma": [_I, _I64, _I, _P, _P],
@@ -174,6 +178,37 @@ def ptr(tensor: torch.Tensor | None) -> int | None:
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+class Route(NamedTuple):
+    """The kernel a GEMM of some shape runs (the ``kq_*_route`` entries)."""
+
+    kernel: str  # generic, stream, panel, tile or square
+    tiles: int   # 16-row weight tiles of a workgroup
+    waves: int
+    splits: int  # K splits over workgroups
+
+
+_ROUTES = ("generic", "stream", "panel", "tile", "square")
+
+
+def _route(entry: str, *args) -> Route:
+    out = (ctypes.c_int32 * 4)()
+    call(entry, *args, ctypes.addressof(out))
+    return Route(_ROUTES[out[0]], out[1], out[2], out[3])
+
+
+def w8a8_route(m: int, n: int, k: int, swiglu: bool = False) -> Route:
+    return _route("kq_w8a8_route", m, n, k, int(swiglu))
+
+
+def block_fp8_route(m: int, n: int, k: int, swiglu: bool = False) -> Route:
+    return _route("kq_block_fp8_route", m, n, k, int(swiglu))
+
+
+def w4a16_route(dtype: torch.dtype, gathered: bool, m: int, n: int, k: int, group_size: int,
+                swiglu: bool = False) -> Route:
+    return _route("kq_w4a16_route", dtype_code(dtype), int(gathered), m, n, k, group_size, int(swiglu))
 
 
 def stream_handle(device: torch.device) -> int:

@@ -116,6 +116,24 @@ extern "C" int kq_block_fp8_gemm(const uint8_t* xq, const float* xs, const uint8
   return check_launch("kq_block_fp8_gemm");
 }
 
+extern "C" int kq_block_fp8_route(int64_t m, int64_t n, int64_t k, int swiglu, int32_t* route) {
+  if (m < 1 || (swiglu && m > 128) || !route || block_check_shape("kq_block_fp8_route", m, n, k) != KQ_OK) {
+    if (m < 1 || (swiglu && m > 128) || !route) set_error("kq_block_fp8_route: bad shape m=%lld", (long long)m);
+    return KQ_EINVAL;
+  }
+  route[3] = 1;
+  if (m <= 64) {
+    const SgForm f = block_raw_applies(m, k) ? sg_raw_form(m, n, (int)k, swiglu)
+                                             : sg_quantized_form(m, n, (int)k, swiglu);
+    route[0] = KQ_ROUTE_STREAM; route[1] = f.nt; route[2] = f.nw;
+  } else if (m <= 256) {
+    route[0] = KQ_ROUTE_PANEL; route[1] = pg_block_tiles(m, n, swiglu); route[2] = 4;
+  } else {
+    route[0] = KQ_ROUTE_TILE; route[1] = 16; route[2] = 8;
+  }
+  return KQ_OK;
+}
+
 extern "C" size_t kq_block_fp8_workspace_size(int64_t m, int64_t k) {
   return m > 0 && k > 0 ? block_quant_bytes(m, k) : 0;
 }

@@ -278,7 +278,7 @@ __global__ void __launch_bounds__(64 * WM) panel_gemm_kernel(PanelArgs pa) {
 // ------------------------------------------------------------------ launch
 struct PanelForm {
   int nt;      // weight tiles per panel
-  int mtw, wm; // row tiles per wave, waves
+  int mtw;     // row tiles per wave (4 waves at nt = 4, else 8)
   int splits;
 };
 
@@ -301,17 +301,17 @@ static inline PanelForm pg_form(int64_t M, int64_t tiles, int KB) {
   if (panels(8) > cus / 2) {
     int nt = panels(8) <= cus ? 8 : 0;
     if (nt == 0 && M <= 128) nt = panels(12) <= cus ? 12 : panels(16) <= cus ? 16 : 0;
-    return PanelForm{nt, big_m, 8, 1};
+    return PanelForm{nt, big_m, 1};
   }
   if (KB >= 64) {
     const int s = (int)std::min<int64_t>(8, cus / panels(8));
-    return PanelForm{8, big_m, 8, s};
+    return PanelForm{8, big_m, s};
   }
   const int64_t units = panels(4) * ((M + 127) / 128);
-  if (M > 128 && units > cus) return PanelForm{0, 0, 0, 1};
+  if (M > 128 && units > cus) return PanelForm{0, 0, 1};
   int s = 1;
   if (units < 96) s = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(4, cus / units), KB / 7));
-  return PanelForm{4, 2, 4, s};
+  return PanelForm{4, 2, s};
 }
 
 template <int FMT, int MTW, int WM, int NT, int R, bool SW>
@@ -339,22 +339,27 @@ static void pg_launch(const PanelArgs& a, const PanelForm& f, hipStream_t stream
 // N = K = 4096 19.0 with 2 tiles, 24.7 with 4 (the tile engine 51); 24576 rows
 // K = 4096 63.9 with 8.  Every form adds an element's K blocks in one order, so
 // a SwiGLU launch gives the bits of its two projections.
+static inline int pg_block_tiles(int64_t m, int64_t n, bool sw) {
+  auto units = [&](int nt) {
+    const int cols = (sw ? 8 : 16) * nt;
+    return (n + cols - 1) / cols * ((m + 127) / 128);
+  };
+  const int64_t need = tg_device_cus() / 2;
+  return units(8) >= need ? 8 : units(4) >= need ? 4 : 2;
+}
 template <bool SW>
 static inline void pg_launch_block(const StreamArgs& s, hipStream_t stream) {
   const PanelArgs a{s, 1, nullptr};
-  const int64_t need = tg_device_cus() / 2, row_tiles = (s.M + 127) / 128;
-  auto units = [&](int nt) {
-    const int cols = (SW ? 8 : 16) * nt;
-    return (s.N + cols - 1) / cols * row_tiles;
-  };
-  if (units(8) >= need) pg_launch_form<kSgBlock, 2, 4, 8, 3, SW>(a, stream);
-  else if (units(4) >= need) pg_launch_form<kSgBlock, 2, 4, 4, 4, SW>(a, stream);
+  const int nt = pg_block_tiles(s.M, s.N, SW);
+  if (nt == 8) pg_launch_form<kSgBlock, 2, 4, 8, 3, SW>(a, stream);
+  else if (nt == 4) pg_launch_form<kSgBlock, 2, 4, 4, 4, SW>(a, stream);
   else pg_launch_form<kSgBlock, 2, 4, 2, 4, SW>(a, stream);
 }
 
-// 33 to 64 rows against many weight tiles: panels of 4 tiles, several
-// workgroups per CU (FP8, M = 64, SwiGLU I = 14336 K = 4096 30.9 us, the
+// 33 to 64 rows against more than two weight tiles per CU: panels of 4 tiles,
+// several workgroups per CU (FP8, M = 64, SwiGLU I = 14336 K = 4096 30.9 us, the
 // streaming kernel 41.3; I = 18944 K = 3584 39.0 and 51.2).
+static inline bool pg_64_applies(int64_t m, int64_t tiles) { return m > 32 && tiles > 2 * (int64_t)tg_device_cus(); }
 template <int FMT, bool SW>
 static void pg_launch_64(const PanelArgs& a, hipStream_t stream) {
   pg_launch_form<FMT, 1, 4, 4, 3, SW>(a, stream);

@@ -518,10 +518,20 @@ __global__ void __launch_bounds__(64 * NW) stream_gemm_kernel(StreamArgs a) {
 // 8 waves at M = 8, and 26.8 / 36.8 / 30.0 at M = 32.  The form depends on the
 // row tiles, `tiles` and K alone, and a SwiGLU pack has as many tiles as its
 // packed linear, so both add the K blocks in one order.
-enum { kSgFew = 0, kSgOne = 1, kSgTwo = 2, kSgMany = 3 };
-static inline int sg_form(int64_t tiles, int K) {
+struct SgForm {
+  int nt, nw;  // weight tiles and waves of a workgroup
+};
+// mt: row tiles of 16; few: the launch has the form of 16 waves.
+static inline SgForm sg_form(int64_t tiles, int K, int mt, bool few) {
   const int64_t cus = tg_device_cus();
-  return 2 * tiles <= cus && K >= 16 * 128 ? kSgFew : tiles <= cus ? kSgOne : tiles <= 2 * cus ? kSgTwo : kSgMany;
+  if (few && 2 * tiles <= cus && K >= 16 * 128) return SgForm{1, 16};
+  const int nw = mt <= 2 ? 8 : 4;
+  return tiles <= cus ? SgForm{1, nw} : tiles <= 2 * cus ? SgForm{2, nw} : SgForm{2, nw / 2};
+}
+static inline int64_t sg_tiles(int64_t n, bool sw) { return sw ? (n + 7) / 8 : (n + 15) / 16; }
+// Form of a launch on quantized rows (at most 64) of n columns (SwiGLU: I).
+static inline SgForm sg_quantized_form(int64_t m, int64_t n, int K, bool sw) {
+  return sg_form(sg_tiles(n, sw), K, (int)((m + 15) / 16), m <= 16);
 }
 
 template <int FMT, bool RAW, int MT, int NT, int NW, int R, int XH, bool SW, int DT>
@@ -532,20 +542,20 @@ static void sg_launch_form(const StreamArgs& a, int row_tiles, hipStream_t strea
 }
 
 template <int FMT, bool RAW, int MT, int XH, bool SW, int DT>
-static void sg_launch_rows(const StreamArgs& a, int form, int row_tiles, hipStream_t stream) {
+static void sg_launch_rows(const StreamArgs& a, SgForm f, int row_tiles, hipStream_t stream) {
   if constexpr (MT == 1 && XH == 1) {
-    if (form == kSgFew) {
+    if (f.nw == 16) {
       sg_launch_form<FMT, RAW, MT, 1, 16, 2, XH, SW, DT>(a, row_tiles, stream);
       return;
     }
   }
   if constexpr (MT <= 2) {
-    if (form <= kSgOne) sg_launch_form<FMT, RAW, MT, 1, 8, 2, XH, SW, DT>(a, row_tiles, stream);
-    else if (form == kSgTwo) sg_launch_form<FMT, RAW, MT, 2, 8, 2, XH, SW, DT>(a, row_tiles, stream);
+    if (f.nt == 1) sg_launch_form<FMT, RAW, MT, 1, 8, 2, XH, SW, DT>(a, row_tiles, stream);
+    else if (f.nw == 8) sg_launch_form<FMT, RAW, MT, 2, 8, 2, XH, SW, DT>(a, row_tiles, stream);
     else sg_launch_form<FMT, RAW, MT, 2, 4, 2, XH, SW, DT>(a, row_tiles, stream);
   } else {
-    if (form <= kSgOne) sg_launch_form<FMT, RAW, MT, 1, 4, 3, XH, SW, DT>(a, row_tiles, stream);
-    else if (form == kSgTwo) sg_launch_form<FMT, RAW, MT, 2, 4, 3, XH, SW, DT>(a, row_tiles, stream);
+    if (f.nt == 1) sg_launch_form<FMT, RAW, MT, 1, 4, 3, XH, SW, DT>(a, row_tiles, stream);
+    else if (f.nw == 4) sg_launch_form<FMT, RAW, MT, 2, 4, 3, XH, SW, DT>(a, row_tiles, stream);
     else sg_launch_form<FMT, RAW, MT, 2, 2, 2, XH, SW, DT>(a, row_tiles, stream);
   }
 }
@@ -553,7 +563,7 @@ static void sg_launch_rows(const StreamArgs& a, int form, int row_tiles, hipStre
 // Quantized activations of a.M <= 64 rows.
 template <int FMT, bool SW>
 static void sg_launch(const StreamArgs& a, hipStream_t stream) {
-  const int form = sg_form((a.N + (SW ? 7 : 15)) / (SW ? 8 : 16), a.K);
+  const SgForm form = sg_quantized_form(a.M, a.N, a.K, SW);
   constexpr int DT = KQ_DTYPE_BF16;
   if (a.M <= 16) sg_launch_rows<FMT, false, 1, 1, SW, DT>(a, form, 1, stream);
   else if (a.M <= 32) sg_launch_rows<FMT, false, 2, 1, SW, DT>(a, form, 1, stream);
@@ -561,11 +571,16 @@ static void sg_launch(const StreamArgs& a, hipStream_t stream) {
   else sg_launch_rows<FMT, false, 4, 1, SW, DT>(a, form, 1, stream);
 }
 
-// fp16 / bf16 activations quantized in the launch: INT8 and FP8 one row,
-// block FP8 up to 16.
+// Form of a launch that quantizes its rows: INT8 and FP8 one row, block FP8
+// up to 16.
+static inline SgForm sg_raw_form(int64_t m, int64_t n, int K, bool sw) {
+  return sg_form(sg_tiles(n, sw), K, 1, m <= 8);
+}
+
+// fp16 / bf16 activations quantized in the launch.
 template <int FMT, bool SW>
 static void sg_launch_raw(const StreamArgs& a, int x_dtype, hipStream_t stream) {
-  const int form = sg_form((a.N + (SW ? 7 : 15)) / (SW ? 8 : 16), a.K);
+  const SgForm form = sg_raw_form(a.M, a.N, a.K, SW);
   if constexpr (FMT == kSgBlock) {
     if (a.M > 8) {
       if (x_dtype == KQ_DTYPE_BF16) sg_launch_rows<FMT, true, 1, 2, SW, KQ_DTYPE_BF16>(a, form, 1, stream);

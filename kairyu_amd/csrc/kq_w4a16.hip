@@ -2045,6 +2045,33 @@ extern "C" int kq_w4a16_tiled_gemm(const void* x, int x_dtype, const int32_t* ti
                 workspace, workspace_bytes, (hipStream_t)stream);
 }
 
+extern "C" int kq_w4a16_route(int x_dtype, int gathered, int64_t m, int64_t n, int64_t k, int group_size,
+                              int swiglu, int32_t* route) {
+  if (m < 1 || n < 8 || n % 8 != 0 || k < 8 || k % 8 != 0 || group_size < 8 || m > 0x7fffffff || n > 0x7fffffff ||
+      k > 0x7fffffff || (swiglu && n % 32 != 0) || !route) {
+    set_error("kq_w4a16_route: bad shape m=%lld n=%lld k=%lld", (long long)m, (long long)n, (long long)k);
+    return KQ_EINVAL;
+  }
+  W4Args a{};
+  a.layout = kLayoutTiles;
+  a.x_dtype = x_dtype;
+  a.M = (int)m; a.N = (int)n; a.K = (int)k; a.G = group_size; a.ldx = (int)k;
+  a.swiglu = swiglu;
+  const int gmode = gathered ? kGroupsPermuted : kGroupsUniform;
+  route[0] = KQ_ROUTE_GENERIC;
+  route[1] = route[2] = 0;
+  route[3] = 1;
+  if (!prefill_applies(a, gmode)) return KQ_OK;
+  W4StreamForm f{};
+  const int ks = prefill_splits(a, (size_t)-1);
+  if (stream_form(a, gmode, ks, &f)) {
+    route[0] = KQ_ROUTE_STREAM; route[1] = f.nt; route[2] = 4; route[3] = f.ksplit;
+  } else {
+    route[0] = KQ_ROUTE_TILE; route[3] = ks;
+  }
+  return KQ_OK;
+}
+
 // Packed gate/up projection with SwiGLU (layers.py:243-244): the tiled operand
 // covers 2I columns, 16-column blocks of gate and up alternating.  Decode
 // shapes run the GEMV with the SwiGLU epilogue; others the tiled GEMM into

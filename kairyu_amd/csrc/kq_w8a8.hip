@@ -23,6 +23,8 @@
 #include "kq_stream_gemm.h"
 #include "kq_tile_gemm.h"
 
+#include <cstring>
+
 namespace kq {
 
 enum { kFmtI8 = 0, kFmtFp8 = 1 };
@@ -51,7 +53,7 @@ struct Epi {
   int out_dtype;
   int32_t* acc_out;
   int M, N;
-  // M <= 64 only: N = 2I packed gate / up weight rows [gate; up], the
+  // streaming and panel kernels: N = 2I packed gate / up weight rows [gate; up], the
   // output out[M][I] = silu(gate) * up (SwiGLU epilogue); 0: out[M][N]
   int swiglu;
 };
@@ -229,7 +231,7 @@ static void launch_stream(const uint8_t* xq, const uint8_t* w, int K, const Epi&
   constexpr int SF = FMT == kFmtI8 ? kSgI8 : kSgFp8;
   StreamArgs a = stream_args(w, K, ep);
   a.x = xq; a.x_bytes = (uint32_t)((int64_t)ep.M * K); a.xs = ep.xscale;
-  if (ep.M > 32 && sg_form((ep.N + 15) / 16, K) == kSgMany) {
+  if (pg_64_applies(ep.M, (ep.N + 15) / 16)) {
     const PanelArgs p{a, 1, nullptr};
     if (ep.swiglu) pg_launch_64<SF, true>(p, stream);
     else pg_launch_64<SF, false>(p, stream);
@@ -242,7 +244,7 @@ static void launch_stream(const uint8_t* xq, const uint8_t* w, int K, const Epi&
 // 65 to 256 rows: the panel kernel's form, nt = 0 where the tile engine or
 // the 128x128 kernel runs instead.
 static PanelForm panel_form(int64_t m, int64_t n, int64_t k) {
-  if (m <= 64 || m > 256 || k % 16 != 0 || k > 65536) return PanelForm{0, 0, 0, 1};
+  if (m <= 64 || m > 256 || k % 16 != 0 || k > 65536) return PanelForm{0, 0, 1};
   return pg_form(m, (n + 15) / 16, (int)((k + 127) / 128));
 }
 
@@ -433,6 +435,30 @@ extern "C" size_t kq_w8a8_workspace_size(int64_t m, int64_t n, int64_t k) {
   const PanelForm panel = panel_form(m, n, k);
   const int s = std::max(panel.nt ? panel.splits : 1, tile_engine_splits(m, n, (int)k, (const void*)1, (size_t)-1));
   return s > 1 ? plane * (size_t)s : 0;
+}
+
+extern "C" int kq_w8a8_route(int64_t m, int64_t n, int64_t k, int swiglu, int32_t* route) {
+  if (m < 1 || n < 1 || k < 1 || m > 0x7fffffff || n > 0x7fffffff || k > 65536 || (swiglu && n % 2) || !route) {
+    set_error("kq_w8a8_route: bad shape m=%lld n=%lld k=%lld", (long long)m, (long long)n, (long long)k);
+    return KQ_EINVAL;
+  }
+  const int K = (int)k;
+  const PanelForm panel = panel_form(m, n, k);
+  int32_t r[4] = {KQ_ROUTE_GENERIC, 0, 0, 1};
+  if (K % 16 != 0) {
+  } else if (m <= 64 && pg_64_applies(m, (n + 15) / 16)) {
+    r[0] = KQ_ROUTE_PANEL; r[1] = 4; r[2] = 4;
+  } else if (m <= 64) {
+    const SgForm f = sg_quantized_form(m, swiglu ? n / 2 : n, K, swiglu);
+    r[0] = KQ_ROUTE_STREAM; r[1] = f.nt; r[2] = f.nw;
+  } else if (panel.nt) {
+    r[0] = KQ_ROUTE_PANEL; r[1] = panel.nt; r[2] = panel.nt == 4 ? 4 : 8; r[3] = panel.splits;
+  } else {
+    const int s = tile_engine_splits(m, n, K, (const void*)1, (size_t)-1);
+    r[0] = s ? KQ_ROUTE_TILE : KQ_ROUTE_SQUARE; r[1] = s ? 16 : 8; r[2] = s ? 8 : 4; r[3] = s ? s : 1;
+  }
+  memcpy(route, r, sizeof(r));
+  return KQ_OK;
 }
 
 extern "C" int kq_w8a8_i8_gemm(const int8_t* xq, const float* xscale, const int8_t* w,

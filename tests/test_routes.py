@@ -1,0 +1,38 @@
+"""Which kernel and form a GEMM of a shape takes: the rules of the dispatch,
+asked of the library without a GPU (256 CUs are assumed then, as on MI355X)."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from kairyu_amd._native import Route, block_fp8_route, w4a16_route, w8a8_route
+
+
+@pytest.fixture(autouse=True)
+def _cus():
+    if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines are stated for 256 CUs")
+
+
+def test_kernels_by_rows():
+    assert w8a8_route(8, 4096, 4100).kernel == "generic"        # K % 16
+    assert w8a8_route(8, 4096, 4096) == Route("stream", 1, 8, 1)
+    assert w8a8_route(8, 28672, 4096) == Route("stream", 2, 4, 1)
+    assert w8a8_route(64, 28672, 4096, swiglu=True) == Route("panel", 4, 4, 1)
+    assert w8a8_route(128, 28672, 4096) == Route("panel", 8, 8, 1)
+    assert w8a8_route(4096, 14336, 4096).kernel == "tile"
+    assert block_fp8_route(8, 4096, 4096) == Route("stream", 1, 8, 1)
+    assert block_fp8_route(257, 4096, 4096).kernel == "tile"
+    assert w4a16_route(torch.float16, False, 16, 4096, 4096, 128).kernel == "generic"
+    assert w4a16_route(torch.float16, False, 32, 4096, 4096, 128) == Route("stream", 4, 4, 4)
+    assert w4a16_route(torch.float16, False, 32, 4096, 4096, 64).kernel == "generic"
+    assert w4a16_route(torch.bfloat16, False, 64, 4096, 4096, 128).kernel == "tile"
+
+
+def test_bad_shapes_are_refused():
+    for call in (lambda: w8a8_route(0, 16, 16), lambda: block_fp8_route(8, 16, 100),
+                 lambda: block_fp8_route(129, 256, 256, swiglu=True),
+                 lambda: w4a16_route(torch.float16, False, 8, 12, 128, 128)):
+        with pytest.raises(ValueError, match="bad shape"):
+            call()
