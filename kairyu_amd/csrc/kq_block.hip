@@ -10,7 +10,8 @@
 //     227.3, 5120 / 6912 (a shard) 186.4 -> 168.6 / 224.1 -> 197.3; at 200 rows
 //     4096 / 12288 lost 2% (276.4 -> 281.0), its two row tiles reading the
 //     activations once per 64 columns and not once per 128.
-//   * M > 256: the persistent tile engine of kq_tile_gemm.h.
+//   * M > 256, or more columns than one round of panels holds
+//     (pg_block_applies): the persistent tile engine of kq_tile_gemm.h.
 #include "kq_common.h"
 #include "kq_panel_gemm.h"
 #include "kq_stream_gemm.h"
@@ -99,7 +100,7 @@ extern "C" int kq_block_fp8_gemm(const uint8_t* xq, const float* xs, const uint8
   }
   const int bad = block_check_shape("kq_block_fp8_gemm", m, n, k);
   if (bad != KQ_OK || m == 0) return bad;
-  if (m <= 256) {
+  if (m <= 256 && pg_block_applies(m, n)) {
     StreamArgs a = block_stream_args(w, ws, bias, bias_dtype, out, out_dtype, m, n, k);
     block_quantized(a, xq, xs);
     block_launch<false>(a, (hipStream_t)stream);
@@ -122,14 +123,14 @@ extern "C" int kq_block_fp8_route(int64_t m, int64_t n, int64_t k, int swiglu, i
     return KQ_EINVAL;
   }
   route[3] = 1;
-  if (m <= 64) {
+  if (m > 256 || !(swiglu || pg_block_applies(m, n))) {
+    route[0] = KQ_ROUTE_TILE; route[1] = 16; route[2] = 8;
+  } else if (m <= 64) {
     const SgForm f = block_raw_applies(m, k) ? sg_raw_form(m, n, (int)k, swiglu)
                                              : sg_quantized_form(m, n, (int)k, swiglu);
     route[0] = KQ_ROUTE_STREAM; route[1] = f.nt; route[2] = f.nw;
-  } else if (m <= 256) {
-    route[0] = KQ_ROUTE_PANEL; route[1] = pg_block_tiles(m, n, swiglu); route[2] = 4;
   } else {
-    route[0] = KQ_ROUTE_TILE; route[1] = 16; route[2] = 8;
+    route[0] = KQ_ROUTE_PANEL; route[1] = pg_block_tiles(m, n, swiglu); route[2] = 4;
   }
   return KQ_OK;
 }

@@ -334,11 +334,24 @@ static void pg_launch(const PanelArgs& a, const PanelForm& f, hipStream_t stream
   }
 }
 
+// Whether block FP8 rows (at most 256) of an unfused product run here or in
+// the streaming kernel; else the tile engine.  A panel of 8 tiles takes a CU's
+// LDS, so past one round of them the second is paid in full: N = 16384 /
+// 16512, M = 256, us, panels against tile engine, K = 2048 31 / 40 and 53 / 40,
+// K = 4096 50 / 70 and 90 / 71, K = 8192 88 / 127 and 158 / 126; N = 32768 /
+// 33024, M = 128, K = 4096 51 / 68 and 88 / 68.  The streaming kernel meets the
+// tile engine later: N = 37888 / 57344 (296 and 448 panels), M = 64, K = 4096
+// 62 / 65 and 81 / 74, M = 49 56 / 64 and 73 / 73.
+static inline bool pg_block_applies(int64_t m, int64_t n) {
+  const int64_t panels = (n + 127) / 128, cus = tg_device_cus();
+  return m <= 48 || (m <= 64 ? 2 * panels <= 3 * cus : panels * ((m + 127) / 128) <= cus);
+}
+
 // Block FP8, 65 to 256 rows (no split K): panels of 8, 4 or 2 tiles against
-// 128 rows, the widest that gives half the CUs a workgroup.  M = 200, us:
-// N = K = 4096 19.0 with 2 tiles, 24.7 with 4 (the tile engine 51); 24576 rows
-// K = 4096 63.9 with 8.  Every form adds an element's K blocks in one order, so
-// a SwiGLU launch gives the bits of its two projections.
+// 128 rows, the widest that gives half the CUs a workgroup.  M = 200, us, with
+// the quantizer: N = K = 4096 30.5 with 2 tiles (the tile engine 66); 12288
+// rows K = 4096 47.7 with 8 (68).  Every form adds an element's K blocks in
+// one order, so a SwiGLU launch gives the bits of its two projections.
 static inline int pg_block_tiles(int64_t m, int64_t n, bool sw) {
   auto units = [&](int nt) {
     const int cols = (sw ? 8 : 16) * nt;

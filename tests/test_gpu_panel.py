@@ -97,3 +97,15 @@ def test_block_fp8_swiglu_panels_give_the_two_pass_bits(cuda, m, width, k, bias,
     _native.call("kq_swiglu", packed.data_ptr(), packed.stride(0), 0, _native.dtype_code(dtype), two.data_ptr(),
                  m, width, _native.stream_handle(cuda))
     assert np.array_equal(bits(mlp(x)), bits(two))
+
+
+# the columns of one round of panels, and a ragged panel more: the tile engine
+@pytest.mark.parametrize("m,n,kernel", [(256, 16384, "panel"), (200, 16440, "tile"), (65, 32768, "panel"),
+                                        (128, 32776, "tile"), (50, 49152, "stream"), (64, 49160, "tile")])
+def test_block_fp8_on_both_sides_of_a_round(cuda, m, n, kernel):
+    banner(f"block fp8 round m={m} n={n}")
+    k = 256
+    assert _native.block_fp8_route(m, n, k).kernel == kernel
+    module = _fill(BlockFp8Linear(k, n, True), _gen(n)).to(cuda)
+    x = torch.randn(m, k, generator=_gen(m)).to(torch.bfloat16)
+    check_block_fp8(module(x.to(cuda)), x, module, label=f"m={m} n={n}")

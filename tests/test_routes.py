@@ -36,3 +36,12 @@ def test_bad_shapes_are_refused():
                  lambda: w4a16_route(torch.float16, False, 8, 12, 128, 128)):
         with pytest.raises(ValueError, match="bad shape"):
             call()
+
+
+@pytest.mark.parametrize("m,most", [(65, 32768), (128, 32768), (129, 16384), (256, 16384), (64, 49152), (49, 49152)])
+def test_block_fp8_panels_stay_within_a_round(m, most):
+    """Past one round of 128-column panels over the CUs (streamed rows: one and
+    a half) the tile engine is the faster one."""
+    assert block_fp8_route(m, most, 2048).kernel in ("panel", "stream")
+    assert block_fp8_route(m, most + 8, 2048).kernel == "tile"
+    assert block_fp8_route(48, 100000, 2048).kernel == "stream"
