@@ -285,15 +285,22 @@ struct PanelForm {
 // Form for M rows (65 to 256) of `tiles` 16-row weight tiles and KB K blocks;
 // nt = 0: another kernel.  One round of workgroups over most CUs at the widest
 // panel that gives it, since a panel's activations are copied once: 8 tiles,
-// and up to 128 rows 12 or 16 where those of 8 are more than the CUs; few
-// tiles take panels of 4 against 128 rows, and long K or few units split K.
-// Beyond 128 rows wider panels only match the tile engine (I = 18944 K = 3584
-// M = 200 68.7 us with 12 tiles, 67.0), and so do two units of 4 tiles per CU
-// (N = 12288 K = 4096 46.4, 40.3).  Measured, FP8 with its quantizer (us; M =
-// 128 / 200, the kernels before in brackets): N = K = 4096 17.6 / 25.8 [28.9 /
-// 30.5], N = 1024 K = 4096 14.9 / 15.8 [22.0 / 25.8], N = 3584 K = 18944 33.6 /
-// 40.1 [49.7 / 54.9], SwiGLU I = 14336 K = 4096 40.0 / 53.4 [59.9 / 70.8],
-// I = 18944 K = 3584 43.2 [65.4].
+// and up to 128 rows 12 or 16 where those of 8 are more than the CUs.  (Beyond
+// 128 rows wider panels only match the tile engine: I = 18944 K = 3584 M = 200
+// 68.7 us with 12 tiles, 67.0.)
+//
+// Fewer panels than half the CUs: panels of 4 tiles against 128 rows, split
+// over K while that leaves CUs idle, with at least 7 K blocks each, 8 where the
+// halves fill the CUs (N = 4096 M = 256, K = 1792 17.9 us whole and 18.5 in two
+// of 7, K = 3072 23.9 and 22.2); panels of 8 tiles split
+// over K where K is long, 64 blocks, or 40 where the panels of 4 are more than
+// half the CUs and would run unsplit (N = 4096 M = 256 K = 4096 / 6144 / 8192 in
+// panels of 4, split in two, against 8: 23.9 / 30.2 / 34.9 and 27.2 / 30.0 /
+// 31.7; N = 6912 K = 5120 M = 190 unsplit 34.4, panels of 8 split 4 ways 31.0,
+// but N = 8192 K = 3072 M = 256 25.1 and 31.8).  Measured, INT8 with its
+// quantizer (us, weights out of cache; the tile engine in brackets): N = K =
+// 4096 M = 128 / 256 18.7 / 23.9 [29 / 34], N = 3456 K = 5120 M = 129 23.6 [30],
+// N = 8192 K = 7168 M = 65 / 190 28.8 / 35.3 [38 / 46].
 static inline PanelForm pg_form(int64_t M, int64_t tiles, int KB) {
   const int64_t cus = tg_device_cus();
   const int big_m = M > 128 ? 2 : 1;
@@ -303,15 +310,11 @@ static inline PanelForm pg_form(int64_t M, int64_t tiles, int KB) {
     if (nt == 0 && M <= 128) nt = panels(12) <= cus ? 12 : panels(16) <= cus ? 16 : 0;
     return PanelForm{nt, big_m, 1};
   }
-  if (KB >= 64) {
-    const int s = (int)std::min<int64_t>(8, cus / panels(8));
-    return PanelForm{8, big_m, s};
-  }
   const int64_t units = panels(4) * ((M + 127) / 128);
+  if (KB >= (2 * units <= cus ? 64 : 40)) return PanelForm{8, big_m, (int)std::min<int64_t>(8, cus / panels(8))};
   if (M > 128 && units > cus) return PanelForm{0, 0, 1};
-  int s = 1;
-  if (units < 96) s = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(4, cus / units), KB / 7));
-  return PanelForm{4, 2, s};
+  const int64_t s = std::min<int64_t>({4, cus / units, KB / (units < 96 ? 7 : 8)});
+  return PanelForm{4, 2, (int)std::max<int64_t>(1, s)};
 }
 
 template <int FMT, int MTW, int WM, int NT, int R, bool SW>

@@ -1,6 +1,7 @@
 """The panel GEMM (65 to 256 rows; from 33 with many weight rows) at the edges
 of its forms: one and two row tiles per wave, panels of 2 to 16 weight tiles,
-split K, K tails, ragged rows and columns, waves without rows."""
+split K, K tails, ragged rows and columns, waves without rows.  Each case says
+which form it means and asks the dispatch."""
 
 from __future__ import annotations
 
@@ -19,15 +20,26 @@ from test_gpu_stream import _fill, _gen
 
 pytestmark = pytest.mark.gpu
 
-# (m, n, k): panels of 4 (unsplit, then split 3 ways), of 8 split 8 ways with a
-# tail, of 8 unsplit, of 12, of 16; one K block and a tail of 16 bytes
-SHAPES = [(65, 6200, 144), (130, 1004, 2832), (256, 1024, 8208), (96, 17000, 272), (129, 33000, 256),
-          (200, 50008, 128), (128, 8, 112), (40, 8600, 400), (64, 9000, 256)]
+# (m, n, k, panel tiles, K splits), each ragged in rows, columns or K: one and
+# two row tiles per wave, every panel width that a product takes, split and
+# whole; tiles None: past the panels (another kernel)
+SHAPES = [(65, 6200, 144, 4, 1), (130, 1004, 2832, 4, 3), (200, 3500, 1808, 4, 2), (128, 8, 112, 4, 1),
+          (256, 1024, 8208, 8, 8), (130, 4200, 5136, 8, 7), (96, 17000, 272, 8, 1), (250, 16500, 272, 8, 1),
+          (100, 33000, 272, 12, 1), (128, 49300, 144, 16, 1), (40, 8600, 400, 4, 1), (64, 9000, 256, 4, 1),
+          (129, 33000, 256, None, 1), (200, 50008, 128, None, 1)]
 
 
-@pytest.mark.parametrize("m,n,k", SHAPES)
-def test_int8_panels_are_exact(cuda, m, n, k):
+def _expect(route, tiles, splits):
+    if tiles is None:
+        assert route.kernel != "panel"
+    else:
+        assert (route.kernel, route.tiles, route.splits) == ("panel", tiles, splits)
+
+
+@pytest.mark.parametrize("m,n,k,tiles,splits", SHAPES)
+def test_int8_panels_are_exact(cuda, m, n, k, tiles, splits):
     banner(f"panel int8 m={m} n={n} k={k}")
+    _expect(_native.w8a8_route(m, n, k), tiles, splits)
     module = _fill(Int8Linear(k, n, True), _gen(n + k)).to(cuda)
     x = torch.randn(m, k, generator=_gen(m)).to(torch.bfloat16)
     acc = torch.empty(m, n, dtype=torch.int32, device=cuda)
@@ -38,9 +50,10 @@ def test_int8_panels_are_exact(cuda, m, n, k):
     assert np.array_equal(np32(out), want)
 
 
-@pytest.mark.parametrize("m,n,k", SHAPES)
-def test_fp8_panels_match_oracle(cuda, m, n, k):
+@pytest.mark.parametrize("m,n,k,tiles,splits", SHAPES)
+def test_fp8_panels_match_oracle(cuda, m, n, k, tiles, splits):
     banner(f"panel fp8 m={m} n={n} k={k}")
+    _expect(_native.w8a8_route(m, n, k), tiles, splits)
     module = _fill(Fp8Linear(k, n, True), _gen(n + k)).to(cuda)
     x = torch.randn(m, k, generator=_gen(m)).to(torch.float16)
     check_fp8(module(x.to(cuda)), x, module, label=f"m={m} n={n} k={k}")
@@ -56,14 +69,21 @@ def test_block_fp8_panels_match_oracle(cuda, m, n, k):
 
 
 # unsplit and split panels (the reduce pairs the columns), every panel width,
-# widths of odd eighths, rows of one and two row tiles per wave
+# widths of odd eighths, rows of one and two row tiles per wave; 256 rows of
+# 34000 columns are past the panels
 @pytest.mark.parametrize("kind,m,width,k,dtype", [
     ("fp8", 65, 1000, 1024, torch.bfloat16), ("fp8", 200, 520, 8320, torch.float16),
     ("fp8", 130, 9000, 272, torch.bfloat16), ("int8", 256, 17000, 256, torch.float16),
     ("int8", 100, 26000, 144, torch.bfloat16), ("fp8", 50, 5004, 400, torch.bfloat16),
-    ("int8", 64, 4600, 512, torch.float16), ("int8", 129, 1004, 2048, torch.float16)])
+    ("int8", 64, 4600, 512, torch.float16), ("int8", 129, 1004, 2048, torch.float16),
+    ("fp8", 100, 17000, 144, torch.bfloat16), ("int8", 128, 24500, 272, torch.float16),
+    ("fp8", 200, 2200, 5136, torch.bfloat16)])
 def test_swiglu_panels_give_the_two_pass_bits(cuda, kind, m, width, k, dtype):
     banner(f"panel swiglu {kind} m={m} I={width} k={k}")
+    route = _native.w8a8_route(m, 2 * width, k, swiglu=True)
+    forms = {1000: (4, 1), 520: (8, 8), 9000: (8, 1), 26000: (16, 1), 5004: (4, 1), 4600: (4, 1), 1004: (4, 2),
+             24500: (12, 1), 2200: (8, 7), 17000: (12, 1) if m == 100 else (None, 1)}
+    _expect(route, *forms[width])
     make = Fp8Linear if kind == "fp8" else Int8Linear
     g = _gen(width)
     pack = QuantLinearPack.create([_fill(make(k, width, True), g).to(cuda) for _ in range(2)])
