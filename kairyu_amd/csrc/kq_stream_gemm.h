@@ -61,6 +61,9 @@ struct StreamArgs {
   void* out;              // [rows][N]
   int out_dtype;
   int32_t* acc_out;       // INT8, not SW: raw accumulators [M][N], or null
+  int splits;             // SPLIT: blockIdx.z's, and the K blocks of each
+  int split_blocks;
+  uint32_t* partials;     // SPLIT: [splits][M][P] raw accumulators, P = N (SW: 2N, up columns from N)
   int scale_mode;         // RAW INT8, FP8: 0 dynamic, 1 scale_in[0], 2 scale_in[row]
   const float* scale_in;
 };
@@ -200,9 +203,12 @@ template <> struct SgAcc<kSgI8> { using T = i32x4; };
 
 // XH: with RAW block FP8, activation rows present in units of 8 (M <= 8: 1).
 // DT: with RAW, the activations' dtype.
-template <int FMT, bool RAW, int MT, int NT, int NW, int R, int XH, bool SW, int DT>
+// SPLIT (INT8, FP8, quantized rows): blockIdx.z takes a range of the K blocks
+// and stores raw accumulators.
+template <int FMT, bool RAW, int MT, int NT, int NW, int R, int XH, bool SW, int DT, bool SPLIT>
 __global__ void __launch_bounds__(64 * NW) stream_gemm_kernel(StreamArgs a) {
   static_assert(!RAW || MT == 1, "at most one row tile quantizes in the launch");
+  static_assert(!SPLIT || (FMT != kSgBlock && !RAW), "quantized INT8 / FP8 rows split");
   using L = SgLds<FMT, RAW, MT, NT, R, XH, SW>;
   using Acc = typename SgAcc<FMT>::T;
   constexpr bool BLOCK = FMT == kSgBlock;
@@ -254,7 +260,14 @@ __global__ void __launch_bounds__(64 * NW) stream_gemm_kernel(StreamArgs a) {
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
   const uint32_t lds0 = lds_base + wave * L::Wave;
 
-  const int nmy = wave < KB ? (KB - wave + NW - 1) / NW : 0;  // this wave's K blocks
+  // this wave's K blocks: kbeg + i * NW
+  int kbeg = wave, nblocks = KB;
+  if constexpr (SPLIT) {
+    const int lo = (int)blockIdx.z * a.split_blocks;
+    nblocks = min(KB - lo, a.split_blocks);
+    kbeg += lo;
+  }
+  const int nmy = wave < nblocks ? (nblocks - wave + NW - 1) / NW : 0;
   // Block scales of this wave's K blocks (slot i: block wave + i * NW) and the
   // routed rows' sources go through LDS by DMA, ahead of the weights: a load
   // into a register would make the compiler wait for every copy in flight.
@@ -291,7 +304,7 @@ __global__ void __launch_bounds__(64 * NW) stream_gemm_kernel(StreamArgs a) {
   // K tails (K % 128 != 0): the last block's chunks past K are not fetched
   // (zeros), in the weights as in the activations
   auto issue_w = [&](int i, int q, bool none) {
-    const int kb = wave + i * NW;
+    const int kb = kbeg + i * NW;
     const int32_t so = __builtin_amdgcn_readfirstlane(none ? 0 : kb * 128);
     const bool tail = !BLOCK && ktail != 128 && kb == KB - 1;
 #pragma unroll
@@ -337,7 +350,7 @@ __global__ void __launch_bounds__(64 * NW) stream_gemm_kernel(StreamArgs a) {
     if (lane < 16 * MT && row0 + lane < row_end) vxs = (a.gather ? gat[lane] : row0 + lane) * KB * 4;
   }
   auto issue_x = [&](int i, int q, bool none) {
-    const int kb = none ? 0 : wave + i * NW;
+    const int kb = none ? 0 : kbeg + i * NW;
     const uint32_t b = lds0 + q * L::Stage + L::W;
     const int32_t so = __builtin_amdgcn_readfirstlane(kb * (RAW ? 256 : 128));
     const bool tail = !BLOCK && ktail != 128 && kb == KB - 1;
@@ -405,7 +418,7 @@ __global__ void __launch_bounds__(64 * NW) stream_gemm_kernel(StreamArgs a) {
       uint8_t* frag = mine + L::Frag;
       const uint16_t q2 = sg_quant2<FMT, DT>(*(const uint32_t*)(xf + lane * 4), row_s, row_rs, row_ok);
       // zeros past K whatever the scale: 0 / 0 under a given scale of zero is NaN
-      *(uint16_t*)(frag + lane * 2) = (wave + i * NW) * 128 + lane * 2 < K ? q2 : (uint16_t)0;
+      *(uint16_t*)(frag + lane * 2) = (kbeg + i * NW) * 128 + lane * 2 < K ? q2 : (uint16_t)0;
       xf = frag;
     } else if constexpr (RAW) {
       uint8_t* frag = mine + L::Frag;
@@ -475,18 +488,27 @@ __global__ void __launch_bounds__(64 * NW) stream_gemm_kernel(StreamArgs a) {
     const int n = SW ? c0 + 8 * nt + (j & 7) : c0 + 16 * nt + j;
     const bool live = n < a.N && m < row_end;
     float v;
+    const bool up_lane = SW && j >= 8;
+    uint32_t raw;
     if constexpr (FMT == kSgI8) {
       int sum = (int)part[0];
 #pragma unroll
       for (int w2 = 1; w2 < NW; ++w2) sum += (int)part[w2];
-      if (!SW && a.acc_out && live) a.acc_out[(int64_t)m * a.N + n] = sum;
+      raw = (uint32_t)sum;
       v = (float)sum;
     } else {
       v = __uint_as_float(part[0]);
 #pragma unroll
       for (int w2 = 1; w2 < NW; ++w2) v = __fadd_rn(v, __uint_as_float(part[w2]));
+      raw = __float_as_uint(v);
     }
-    const bool up_lane = SW && j >= 8;
+    if constexpr (SPLIT) {
+      if (live) a.partials[((int64_t)blockIdx.z * a.M + m) * (SW ? 2 * a.N : a.N) + (up_lane ? a.N : 0) + n] = raw;
+      continue;
+    }
+    if constexpr (FMT == kSgI8 && !SW) {
+      if (a.acc_out && live) a.acc_out[(int64_t)m * a.N + n] = (int)raw;
+    }
     if (live) {
       if constexpr (!BLOCK) {
         v = __fmul_rn(__fmul_rn(v, RAW ? row_s : epi_xs[m - row0]), epi_ws[(up_lane ? 64 : 0) + n - c0]);
@@ -534,11 +556,11 @@ static inline SgForm sg_quantized_form(int64_t m, int64_t n, int K, bool sw) {
   return sg_form(sg_tiles(n, sw), K, (int)((m + 15) / 16), m <= 16);
 }
 
-template <int FMT, bool RAW, int MT, int NT, int NW, int R, int XH, bool SW, int DT>
+template <int FMT, bool RAW, int MT, int NT, int NW, int R, int XH, bool SW, int DT, bool SPLIT = false>
 static void sg_launch_form(const StreamArgs& a, int row_tiles, hipStream_t stream) {
   constexpr int cols = (SW ? 8 : 16) * NT;
-  const dim3 grid((unsigned)((a.N + cols - 1) / cols), (unsigned)row_tiles);
-  hipLaunchKernelGGL((stream_gemm_kernel<FMT, RAW, MT, NT, NW, R, XH, SW, DT>), grid, dim3(64 * NW), 0, stream, a);
+  const dim3 grid((unsigned)((a.N + cols - 1) / cols), (unsigned)row_tiles, SPLIT ? (unsigned)a.splits : 1u);
+  hipLaunchKernelGGL((stream_gemm_kernel<FMT, RAW, MT, NT, NW, R, XH, SW, DT, SPLIT>), grid, dim3(64 * NW), 0, stream, a);
 }
 
 template <int FMT, bool RAW, int MT, int XH, bool SW, int DT>
@@ -546,6 +568,13 @@ static void sg_launch_rows(const StreamArgs& a, SgForm f, int row_tiles, hipStre
   if constexpr (MT == 1 && XH == 1) {
     if (f.nw == 16) {
       sg_launch_form<FMT, RAW, MT, 1, 16, 2, XH, SW, DT>(a, row_tiles, stream);
+      return;
+    }
+  }
+  if constexpr (FMT != kSgBlock && !RAW && MT >= 2) {
+    if (a.splits > 1) {  // (narrow products: one tile a workgroup)
+      if constexpr (MT == 2) sg_launch_form<FMT, RAW, MT, 1, 8, 2, XH, SW, DT, true>(a, row_tiles, stream);
+      else sg_launch_form<FMT, RAW, MT, 1, 4, 3, XH, SW, DT, true>(a, row_tiles, stream);
       return;
     }
   }

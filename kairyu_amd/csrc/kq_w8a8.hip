@@ -226,8 +226,32 @@ static StreamArgs stream_args(const uint8_t* w, int K, const Epi& ep) {
   return a;
 }
 
+// Adds the raw accumulators of `splits` K ranges in order, with the epilogue.
 template <int FMT>
-static void launch_stream(const uint8_t* xq, const uint8_t* w, int K, const Epi& ep, hipStream_t stream) {
+static void reduce_splits(const void* partials, int splits, const Epi& ep, hipStream_t stream) {
+  ReduceArgs r{partials, splits, ep.M, ep.N, ep.xscale, ep.wscale, ep.ws_per_channel,
+               ep.bias, ep.bias_dtype, ep.out, ep.out_dtype, ep.acc_out, ep.swiglu};
+  launch_splitk_reduce(FMT == kFmtI8 ? kReduceI8 : kReduceFp8, r, stream);
+}
+
+// K splits of a streaming launch (17 to 64 rows) over workgroups.  Narrow
+// products leave most CUs idle, and with long K the few that work walk it
+// alone; a split costs the reduce launch, about 1.5 us.  INT8 with its
+// quantizer, weights out of cache, us, whole / 4 / 8 splits: N = 512 M = 24
+// K = 4096 9.0 / 9.8 / 10.8, K = 8192 12.0 / 11.0 / 11.7, K = 16384 17.1 /
+// 13.0 / 13.1; M = 33 N = 1024 K = 4096 10.1 / 10.7; M = 64 N = 512 12.0 / 11.1 / 12.1, 17.1 / 13.0 / 13.4, 26.4 / 16.6 /
+// 15.6; N = 1536 (whole / 2) M = 17 K = 8192 12.3 / 12.7, K = 12288 15.7 / 14.7.
+static int stream_splits(int64_t m, int64_t n, int64_t k) {
+  const int64_t room = tg_device_cus() / ((n + 15) / 16), kb = (k + 127) / 128;
+  if (m <= 16) return 1;
+  if (room >= 8 && kb >= (m > 32 ? 96 : 128)) return 8;
+  if (room >= 4 && kb >= (m > 48 ? 32 : m > 32 ? 40 : 64)) return 4;
+  return room >= 2 && kb >= 96 ? 2 : 1;
+}
+
+template <int FMT>
+static void launch_stream(const uint8_t* xq, const uint8_t* w, int K, const Epi& ep, void* workspace,
+                          size_t ws_bytes, hipStream_t stream) {
   constexpr int SF = FMT == kFmtI8 ? kSgI8 : kSgFp8;
   StreamArgs a = stream_args(w, K, ep);
   a.x = xq; a.x_bytes = (uint32_t)((int64_t)ep.M * K); a.xs = ep.xscale;
@@ -237,8 +261,13 @@ static void launch_stream(const uint8_t* xq, const uint8_t* w, int K, const Epi&
     else pg_launch_64<SF, false>(p, stream);
     return;
   }
+  a.splits = stream_splits(ep.M, ep.N, K);
+  if (!workspace || (size_t)a.splits * (size_t)ep.M * (size_t)ep.N * 4 > ws_bytes) a.splits = 1;
+  a.split_blocks = ((K + 127) / 128 + a.splits - 1) / a.splits;  // (at least 4: none is empty)
+  a.partials = (uint32_t*)workspace;
   if (ep.swiglu) sg_launch<SF, true>(a, stream);
   else sg_launch<SF, false>(a, stream);
+  if (a.splits > 1) reduce_splits<FMT>(workspace, a.splits, ep, stream);
 }
 
 // 65 to 256 rows: the panel kernel's form, nt = 0 where the tile engine or
@@ -257,11 +286,7 @@ static void launch_panel(const uint8_t* xq, const uint8_t* w, int K, const Epi& 
   p.s.x = xq; p.s.x_bytes = (uint32_t)((int64_t)ep.M * K); p.s.xs = ep.xscale;
   if (ep.swiglu) pg_launch<SF, true>(p, f, stream);
   else pg_launch<SF, false>(p, f, stream);
-  if (f.splits > 1) {
-    ReduceArgs r{workspace, f.splits, ep.M, ep.N, ep.xscale, ep.wscale, ep.ws_per_channel,
-                 ep.bias, ep.bias_dtype, ep.out, ep.out_dtype, ep.acc_out, ep.swiglu};
-    launch_splitk_reduce(FMT == kFmtI8 ? kReduceI8 : kReduceFp8, r, stream);
-  }
+  if (f.splits > 1) reduce_splits<FMT>(workspace, f.splits, ep, stream);
 }
 
 // One fp16 / bf16 row, quantized in the launch.
@@ -336,7 +361,7 @@ static int run_w8a8(const char* what, const uint8_t* xq, const uint8_t* w, int64
     return KQ_EINVAL;
   }
   if (m <= 64 && m * k < ((int64_t)1 << 31) && k < ((int64_t)1 << 26)) {
-    launch_stream<FMT>(xq, w, K, ep, stream);
+    launch_stream<FMT>(xq, w, K, ep, workspace, ws_bytes, stream);
   } else if (panel.nt) {
     launch_panel<FMT>(xq, w, K, ep, panel, workspace, ws_bytes, stream);
   }
@@ -357,9 +382,7 @@ static int run_w8a8(const char* what, const uint8_t* xq, const uint8_t* w, int64
     a.partials = splits > 1 ? (uint32_t*)workspace : nullptr;
     tg_launch<FMT == kFmtI8 ? kTgI8 : kTgFp8, false, kTgEpiStore>(a, stream);
     if (splits > 1) {
-      ReduceArgs r{workspace, splits, ep.M, ep.N, ep.xscale, ep.wscale, ep.ws_per_channel,
-                   ep.bias, ep.bias_dtype, ep.out, ep.out_dtype, ep.acc_out};
-      launch_splitk_reduce(FMT == kFmtI8 ? kReduceI8 : kReduceFp8, r, stream);
+      reduce_splits<FMT>(workspace, splits, ep, stream);
     }
   } else {
     const int tiles_m = (int)((m + kTile - 1) / kTile);
@@ -431,7 +454,10 @@ static int run_linear(const char* what, const void* x, int x_dtype, int64_t ldx,
 extern "C" size_t kq_w8a8_workspace_size(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k <= 0 || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff) return 0;
   const size_t plane = (size_t)m * (size_t)n * 4;
-  if (m <= 64) return 0;  // the weight-streaming kernel splits K within a workgroup only
+  if (m <= 64) {
+    const int s = k % 16 == 0 ? stream_splits(m, n, k) : 1;
+    return s > 1 ? plane * (size_t)s : 0;
+  }
   const PanelForm panel = panel_form(m, n, k);
   const int s = std::max(panel.nt ? panel.splits : 1, tile_engine_splits(m, n, (int)k, (const void*)1, (size_t)-1));
   return s > 1 ? plane * (size_t)s : 0;
@@ -450,7 +476,7 @@ extern "C" int kq_w8a8_route(int64_t m, int64_t n, int64_t k, int swiglu, int32_
     r[0] = KQ_ROUTE_PANEL; r[1] = 4; r[2] = 4;
   } else if (m <= 64) {
     const SgForm f = sg_quantized_form(m, swiglu ? n / 2 : n, K, swiglu);
-    r[0] = KQ_ROUTE_STREAM; r[1] = f.nt; r[2] = f.nw;
+    r[0] = KQ_ROUTE_STREAM; r[1] = f.nt; r[2] = f.nw; r[3] = stream_splits(m, n, k);
   } else if (panel.nt) {
     r[0] = KQ_ROUTE_PANEL; r[1] = panel.nt; r[2] = panel.nt == 4 ? 4 : 8; r[3] = panel.splits;
   } else {

@@ -254,13 +254,17 @@ def test_swiglu_pack_in_a_graph(cuda):
         assert torch.equal(out, eager)
 
 
-@pytest.mark.parametrize("scheme,m,k,width", [("fp8", 16, 4096, 4096), ("fp8", 40, 14336, 1024),
-                                               ("int8", 24, 3584, 2048)])
-def test_w8a8_swiglu_pack_in_a_graph(cuda, scheme, m, k, width):
-    """W8A8 decode / skinny GEMMs with the SwiGLU epilogue (and, at K = 14336,
-    the split-K reduce that pairs the columns) captured once, replayed with
-    eager work between the replays, every replay equal to the eager call."""
+@pytest.mark.parametrize("scheme,m,k,width,splits", [
+    ("fp8", 16, 4096, 4096, 1), ("fp8", 40, 14336, 1024, 2), ("int8", 24, 3584, 2048, 1),
+    ("int8", 40, 8208, 500, 4), ("fp8", 200, 8320, 520, 8)])
+def test_w8a8_swiglu_pack_in_a_graph(cuda, scheme, m, k, width, splits):
+    """W8A8 streaming and panel GEMMs with the SwiGLU epilogue, or with the
+    split-K reduce that pairs the columns, captured once, replayed with eager
+    work between the replays, every replay equal to the eager call."""
 
+    from kairyu_amd._native import w8a8_route
+
+    assert w8a8_route(m, 2 * width, k, swiglu=True).splits == splits
     gate, up = (mod.to(cuda) for mod in _swiglu_pair(scheme, k, width, True, seed=m + k))
     pack = QuantLinearPack.create([gate, up])
     x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).to(torch.bfloat16).to(cuda)

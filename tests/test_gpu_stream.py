@@ -9,6 +9,7 @@ import pytest
 import torch
 
 from gpu_helpers import assert_moe_close, banner, bits, check_block_fp8, check_fp8, np32
+from kairyu_amd._native import w8a8_route
 from kairyu_amd.kernels import quant_gemm_hip as hip
 from kairyu_amd.moe import BlockFp8ExpertMlp, GroupedBlockFp8Experts
 from kairyu_amd.quant.block_fp8 import quantize_block_fp8
@@ -21,9 +22,16 @@ from oracle import moe as omoe
 pytestmark = pytest.mark.gpu
 
 ROWS = [1, 2, 15, 16, 17, 32, 33, 48, 49, 64]
-# one block, a tail of 16 bytes, 19 blocks for 16 waves with a tail; 1 to 600
-# column tiles (16 waves, 8 waves, two tiles, many workgroups per CU)
-SHAPES = [(24, 112), (200, 144), (2600, 2368), (4616, 640), (9608, 272)]
+# one block, a tail of 16 bytes, 19 blocks for 8 and for 16 waves with a tail;
+# 1 to 600 column tiles (one tile, two, many workgroups per CU); long K split
+# over workgroups 4 and 8 ways with a tail
+SHAPES = [(24, 112), (200, 144), (2600, 2368), (1000, 2368), (4616, 640), (9608, 272), (1000, 8272), (72, 16400)]
+
+
+def test_the_shapes_reach_every_form():
+    reached = {w8a8_route(m, n, k)[1:] for m in ROWS for n, k in SHAPES}
+    assert reached >= {(1, 16, 1), (1, 8, 1), (2, 8, 1), (2, 4, 1), (1, 4, 1), (4, 4, 1), (1, 8, 4), (1, 8, 8),
+                       (1, 4, 4), (1, 4, 8)}
 
 
 def _gen(seed):

@@ -6,6 +6,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+from kairyu_amd import _native
 from kairyu_amd._native import Route, block_fp8_route, w4a16_route, w8a8_route
 
 
@@ -55,3 +56,14 @@ def test_block_fp8_panels_stay_within_a_round(m, most):
 def test_w8a8_panels_leave_no_half_of_the_cus_idle(m, n, k, tiles, splits):
     assert w8a8_route(m, n, k) == Route("panel", tiles, 4 if tiles == 4 else 8, splits)
     assert w8a8_route(m, n, k, swiglu=True) == w8a8_route(m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k,splits", [
+    (16, 512, 16384, 1), (17, 512, 8191, 1), (17, 512, 8192, 4), (32, 512, 16384, 8), (33, 512, 4096, 1), (33, 512, 5120, 4),
+    (64, 512, 12288, 8), (64, 1024, 12288, 4), (64, 2048, 8192, 1), (17, 2048, 12288, 2), (64, 2064, 16384, 1),
+    (49, 512, 4096, 4), (64, 512, 3968, 1)])
+def test_few_rows_of_narrow_long_products_split_k(m, n, k, splits):
+    route = w8a8_route(m, n, k)
+    assert route.splits == splits and route.kernel == ("generic" if k % 16 else "stream")
+    need = _native.library().kq_w8a8_workspace_size(m, n, k)
+    assert need == (splits * m * n * 4 if splits > 1 else 0)
