@@ -126,8 +126,8 @@ extern "C" int kq_block_fp8_route(int64_t m, int64_t n, int64_t k, int swiglu, i
   if (m > 256 || !(swiglu || pg_block_applies(m, n))) {
     route[0] = KQ_ROUTE_TILE; route[1] = 16; route[2] = 8;
   } else if (m <= 64) {
-    const SgForm f = block_raw_applies(m, k) ? sg_raw_form(m, n, (int)k, swiglu)
-                                             : sg_quantized_form(m, n, (int)k, swiglu);
+    const SgForm f = block_raw_applies(m, k) ? sg_raw_form(true, m, n, (int)k, swiglu)
+                                             : sg_quantized_form(true, m, n, (int)k, swiglu);
     route[0] = KQ_ROUTE_STREAM; route[1] = f.nt; route[2] = f.nw;
   } else {
     route[0] = KQ_ROUTE_PANEL; route[1] = pg_block_tiles(m, n, swiglu); route[2] = 4;

@@ -527,10 +527,14 @@ __global__ void __launch_bounds__(64 * NW) stream_gemm_kernel(StreamArgs a) {
 
 // ------------------------------------------------------------------ launch
 // Form of a launch over `tiles` 16-row weight tiles: how many of them a
-// workgroup takes (NT) and its waves (NW).  Up to half a tile per CU, one
-// row tile and a K block for each, one tile and 16 waves (M = 1, N = 1024 K = 4096: 4.5 us, 4.9 with
-// 8); up to one tile per CU, one tile and 8 waves, so that every CU streams;
-// up to two, two tiles (one round of
+// workgroup takes (NT) and its waves (NW).  Up to half a tile per CU and one
+// row, one tile and 16 waves: a wave has few K blocks then, and each waits for
+// memory.  (FP8, us, 16 waves against 8: one row N = 1024 K = 4096 4.6 / 4.8, K =
+// 8192 6.4 / 6.8, but N = 256 K = 2048 3.5 / 3.3, a K block a wave; with more
+// rows the waves' sums cost what their loads gain: N = 512 M = 8 K = 4096 6.8 /
+// 6.7, K = 16384 13.7 / 13.1.)  Block FP8 takes 16 waves up to its first 16 rows'
+// form, whose waves quantize, from a K block a wave.  Up to one tile per CU, one
+// tile and 8 waves, so that every CU streams; up to two, two tiles (one round of
 // workgroups); beyond, two tiles and 4 waves, several workgroups per CU, so
 // that one's prologue and epilogue run under another's stream.  Measured, FP8
 // (us; graph replay, weights rotating past the MALL): N = K = 4096 M = 8 5.6,
@@ -544,16 +548,16 @@ struct SgForm {
   int nt, nw;  // weight tiles and waves of a workgroup
 };
 // mt: row tiles of 16; few: the launch has the form of 16 waves.
-static inline SgForm sg_form(int64_t tiles, int K, int mt, bool few) {
+static inline SgForm sg_form(int64_t tiles, int mt, bool few) {
   const int64_t cus = tg_device_cus();
-  if (few && 2 * tiles <= cus && K >= 16 * 128) return SgForm{1, 16};
+  if (few && 2 * tiles <= cus) return SgForm{1, 16};
   const int nw = mt <= 2 ? 8 : 4;
   return tiles <= cus ? SgForm{1, nw} : tiles <= 2 * cus ? SgForm{2, nw} : SgForm{2, nw / 2};
 }
 static inline int64_t sg_tiles(int64_t n, bool sw) { return sw ? (n + 7) / 8 : (n + 15) / 16; }
 // Form of a launch on quantized rows (at most 64) of n columns (SwiGLU: I).
-static inline SgForm sg_quantized_form(int64_t m, int64_t n, int K, bool sw) {
-  return sg_form(sg_tiles(n, sw), K, (int)((m + 15) / 16), m <= 16);
+static inline SgForm sg_quantized_form(bool block, int64_t m, int64_t n, int K, bool sw) {
+  return sg_form(sg_tiles(n, sw), (int)((m + 15) / 16), block ? m <= 16 && K >= 2048 : m == 1 && K > 2048);
 }
 
 template <int FMT, bool RAW, int MT, int NT, int NW, int R, int XH, bool SW, int DT, bool SPLIT = false>
@@ -592,7 +596,7 @@ static void sg_launch_rows(const StreamArgs& a, SgForm f, int row_tiles, hipStre
 // Quantized activations of a.M <= 64 rows.
 template <int FMT, bool SW>
 static void sg_launch(const StreamArgs& a, hipStream_t stream) {
-  const SgForm form = sg_quantized_form(a.M, a.N, a.K, SW);
+  const SgForm form = sg_quantized_form(FMT == kSgBlock, a.M, a.N, a.K, SW);
   constexpr int DT = KQ_DTYPE_BF16;
   if (a.M <= 16) sg_launch_rows<FMT, false, 1, 1, SW, DT>(a, form, 1, stream);
   else if (a.M <= 32) sg_launch_rows<FMT, false, 2, 1, SW, DT>(a, form, 1, stream);
@@ -602,14 +606,14 @@ static void sg_launch(const StreamArgs& a, hipStream_t stream) {
 
 // Form of a launch that quantizes its rows: INT8 and FP8 one row, block FP8
 // up to 16.
-static inline SgForm sg_raw_form(int64_t m, int64_t n, int K, bool sw) {
-  return sg_form(sg_tiles(n, sw), K, 1, m <= 8);
+static inline SgForm sg_raw_form(bool block, int64_t m, int64_t n, int K, bool sw) {
+  return sg_form(sg_tiles(n, sw), 1, block ? m <= 8 && K >= 2048 : K > 2048);
 }
 
 // fp16 / bf16 activations quantized in the launch.
 template <int FMT, bool SW>
 static void sg_launch_raw(const StreamArgs& a, int x_dtype, hipStream_t stream) {
-  const SgForm form = sg_raw_form(a.M, a.N, a.K, SW);
+  const SgForm form = sg_raw_form(FMT == kSgBlock, a.M, a.N, a.K, SW);
   if constexpr (FMT == kSgBlock) {
     if (a.M > 8) {
       if (x_dtype == KQ_DTYPE_BF16) sg_launch_rows<FMT, true, 1, 2, SW, KQ_DTYPE_BF16>(a, form, 1, stream);

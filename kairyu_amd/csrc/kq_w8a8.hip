@@ -237,10 +237,11 @@ static void reduce_splits(const void* partials, int splits, const Epi& ep, hipSt
 // K splits of a streaming launch (17 to 64 rows) over workgroups.  Narrow
 // products leave most CUs idle, and with long K the few that work walk it
 // alone; a split costs the reduce launch, about 1.5 us.  INT8 with its
-// quantizer, weights out of cache, us, whole / 4 / 8 splits: N = 512 M = 24
-// K = 4096 9.0 / 9.8 / 10.8, K = 8192 12.0 / 11.0 / 11.7, K = 16384 17.1 /
-// 13.0 / 13.1; M = 33 N = 1024 K = 4096 10.1 / 10.7; M = 64 N = 512 12.0 / 11.1 / 12.1, 17.1 / 13.0 / 13.4, 26.4 / 16.6 /
-// 15.6; N = 1536 (whole / 2) M = 17 K = 8192 12.3 / 12.7, K = 12288 15.7 / 14.7.
+// quantizer, weights out of cache, us, whole / 4 / 8 splits: N = 512 M = 17
+// K = 4096 9.0 / 9.8 / 10.8, K = 8192 12.0 / 11.0 / 11.7, K = 16384 17.1 / 13.0 /
+// 13.1; M = 33 N = 1024 K = 4096 10.1 / 10.7; M = 64 N = 512 12.0 / 11.1 / 12.1,
+// 17.1 / 13.0 / 13.4, 26.4 / 16.6 / 15.6; N = 1536 (whole / 2) M = 17 K = 8192
+// 12.3 / 12.7, K = 12288 15.7 / 14.7.
 static int stream_splits(int64_t m, int64_t n, int64_t k) {
   const int64_t room = tg_device_cus() / ((n + 15) / 16), kb = (k + 127) / 128;
   if (m <= 16) return 1;
@@ -475,7 +476,7 @@ extern "C" int kq_w8a8_route(int64_t m, int64_t n, int64_t k, int swiglu, int32_
   } else if (m <= 64 && pg_64_applies(m, (n + 15) / 16)) {
     r[0] = KQ_ROUTE_PANEL; r[1] = 4; r[2] = 4;
   } else if (m <= 64) {
-    const SgForm f = sg_quantized_form(m, swiglu ? n / 2 : n, K, swiglu);
+    const SgForm f = sg_quantized_form(false, m, swiglu ? n / 2 : n, K, swiglu);
     r[0] = KQ_ROUTE_STREAM; r[1] = f.nt; r[2] = f.nw; r[3] = stream_splits(m, n, k);
   } else if (panel.nt) {
     r[0] = KQ_ROUTE_PANEL; r[1] = panel.nt; r[2] = panel.nt == 4 ? 4 : 8; r[3] = panel.splits;

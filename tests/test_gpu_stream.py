@@ -22,7 +22,7 @@ from oracle import moe as omoe
 pytestmark = pytest.mark.gpu
 
 ROWS = [1, 2, 15, 16, 17, 32, 33, 48, 49, 64]
-# one block, a tail of 16 bytes, 19 blocks for 8 and for 16 waves with a tail;
+# one block, a tail of 16 bytes, 19 blocks for 8 and (one row) 16 waves with a tail;
 # 1 to 600 column tiles (one tile, two, many workgroups per CU); long K split
 # over workgroups 4 and 8 ways with a tail
 SHAPES = [(24, 112), (200, 144), (2600, 2368), (1000, 2368), (4616, 640), (9608, 272), (1000, 8272), (72, 16400)]

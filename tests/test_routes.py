@@ -67,3 +67,10 @@ def test_few_rows_of_narrow_long_products_split_k(m, n, k, splits):
     assert route.splits == splits and route.kernel == ("generic" if k % 16 else "stream")
     need = _native.library().kq_w8a8_workspace_size(m, n, k)
     assert need == (splits * m * n * 4 if splits > 1 else 0)
+
+
+@pytest.mark.parametrize("m,n,k,waves", [(1, 1024, 4096, 16), (1, 1024, 2048, 8), (1, 2064, 4096, 8),
+                                         (2, 1024, 4096, 8), (16, 512, 16384, 8)])
+def test_sixteen_waves_are_for_one_row(m, n, k, waves):
+    assert w8a8_route(m, n, k).waves == waves
+    assert w8a8_route(m, n, k, swiglu=True) == w8a8_route(m, n, k)
