@@ -290,17 +290,18 @@ struct PanelForm {
 // 68.7 us with 12 tiles, 67.0.)
 //
 // Fewer panels than half the CUs: panels of 4 tiles against 128 rows, split
-// over K while that leaves CUs idle, with at least 7 K blocks each, 8 where the
-// halves fill the CUs (N = 4096 M = 256, K = 1792 17.9 us whole and 18.5 in two
-// of 7, K = 3072 23.9 and 22.2); panels of 8 tiles split
-// over K where K is long, 64 blocks, or 40 where the panels of 4 are more than
-// half the CUs and would run unsplit (N = 4096 M = 256 K = 4096 / 6144 / 8192 in
-// panels of 4, split in two, against 8: 23.9 / 30.2 / 34.9 and 27.2 / 30.0 /
-// 31.7; N = 6912 K = 5120 M = 190 unsplit 34.4, panels of 8 split 4 ways 31.0,
-// but N = 8192 K = 3072 M = 256 25.1 and 31.8).  Measured, INT8 with its
-// quantizer (us, weights out of cache; the tile engine in brackets): N = K =
-// 4096 M = 128 / 256 18.7 / 23.9 [29 / 34], N = 3456 K = 5120 M = 129 23.6 [30],
-// N = 8192 K = 7168 M = 65 / 190 28.8 / 35.3 [38 / 46].
+// over K while that leaves CUs idle, with at least 7 K blocks each, 12 where the
+// halves fill the CUs (N = 4096 M = 256, FP8, K = 2048 17.5 us whole and 18.3 in
+// two of 8; INT8, K = 3072 23.9 and 22.2); panels of 8 tiles split over K where K
+// is long, 64 blocks, or 48 where the panels of 4 are more than half the CUs and
+// would run unsplit, 40 up to 160 rows (N = 4096 M = 256 K = 4096 / 6144 / 8192
+// INT8 in panels of 4, split in two, against 8: 23.9 / 30.2 / 34.9 and 27.2 /
+// 30.0 / 31.7; N = 7168 K = 5120 unsplit against panels of 8 split 4 ways: FP8 M =
+// 129 / 256 30.1 / 33.0 and 28.2 / 35.6, N = 8192 K = 6144 INT8 39.1 / 41.2 and
+// 32.4 / 37.2).  Measured, INT8 with its quantizer (us, weights out of cache; the
+// tile engine in brackets): N = K = 4096 M = 128 / 256 18.7 / 23.9 [29 / 34],
+// N = 3456 K = 5120 M = 129 23.6 [30], N = 8192 K = 7168 M = 65 / 190 28.8 / 35.3
+// [38 / 46].
 static inline PanelForm pg_form(int64_t M, int64_t tiles, int KB) {
   const int64_t cus = tg_device_cus();
   const int big_m = M > 128 ? 2 : 1;
@@ -311,9 +312,9 @@ static inline PanelForm pg_form(int64_t M, int64_t tiles, int KB) {
     return PanelForm{nt, big_m, 1};
   }
   const int64_t units = panels(4) * ((M + 127) / 128);
-  if (KB >= (2 * units <= cus ? 64 : 40)) return PanelForm{8, big_m, (int)std::min<int64_t>(8, cus / panels(8))};
+  if (KB >= (2 * units <= cus ? 64 : M > 128 && M <= 160 ? 40 : 48)) return PanelForm{8, big_m, (int)std::min<int64_t>(8, cus / panels(8))};
   if (M > 128 && units > cus) return PanelForm{0, 0, 1};
-  const int64_t s = std::min<int64_t>({4, cus / units, KB / (units < 96 ? 7 : 8)});
+  const int64_t s = std::min<int64_t>({4, cus / units, KB / (units < 96 ? 7 : 12)});
   return PanelForm{4, 2, (int)std::max<int64_t>(1, s)};
 }
 

@@ -50,9 +50,10 @@ def test_block_fp8_panels_stay_within_a_round(m, most):
 
 @pytest.mark.parametrize("m,n,k,tiles,splits", [
     (129, 3456, 5120, 4, 2), (256, 4096, 7168, 4, 2), (65, 8192, 7168, 4, 2),   # at most half the CUs
-    (129, 5120, 5120, 8, 6), (190, 6912, 5120, 8, 4), (129, 8192, 8064, 8, 4),  # more, 40 K blocks up
+    (129, 5120, 5120, 8, 6), (190, 6912, 6144, 8, 4), (129, 8192, 8064, 8, 4),  # more, long K
+    (190, 6912, 5120, 4, 1), (128, 13824, 5120, 4, 1),
     (256, 8192, 3072, 4, 1), (129, 6144, 4096, 4, 1),                            # more, short K
-    (256, 4096, 1792, 4, 1), (65, 1024, 4096, 4, 4), (200, 1024, 8192, 8, 8)])
+    (256, 4096, 2048, 4, 1), (256, 4096, 3072, 4, 2), (65, 1024, 4096, 4, 4), (200, 1024, 8192, 8, 8)])
 def test_w8a8_panels_leave_no_half_of_the_cus_idle(m, n, k, tiles, splits):
     assert w8a8_route(m, n, k) == Route("panel", tiles, 4 if tiles == 4 else 8, splits)
     assert w8a8_route(m, n, k, swiglu=True) == w8a8_route(m, n, k)
