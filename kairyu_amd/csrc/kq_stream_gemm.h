@@ -9,7 +9,8 @@
 // everything else is arranged around keeping that stream full:
 //   * A workgroup owns 16 * NT output columns; its NW waves take K blocks
 //     (128 bytes of K, one scale block) wave, wave + NW, ...: the waves of a
-//     workgroup stream neighbouring lines of the same weight rows.
+//     workgroup stream neighbouring lines of the same weight rows (but where
+//     the rows' pitch would put those on the same memory channels: sg_apart).
 //   * Every wave keeps a private ring of R stages in LDS, filled by LDS DMA
 //     in whole 128-byte lines (8 rows x 128 B per instruction) and read back
 //     as MFMA fragments through the tile engine's chunk swizzle.  A wave only
@@ -205,10 +206,13 @@ template <> struct SgAcc<kSgI8> { using T = i32x4; };
 // DT: with RAW, the activations' dtype.
 // SPLIT (INT8, FP8, quantized rows): blockIdx.z takes a range of the K blocks
 // and stores raw accumulators.
-template <int FMT, bool RAW, int MT, int NT, int NW, int R, int XH, bool SW, int DT, bool SPLIT>
+// APART (INT8, FP8; NW divides the K blocks): a wave takes neighbouring K
+// blocks, not blocks wave, wave + NW, ...
+template <int FMT, bool RAW, int MT, int NT, int NW, int R, int XH, bool SW, int DT, bool SPLIT, bool APART>
 __global__ void __launch_bounds__(64 * NW) stream_gemm_kernel(StreamArgs a) {
   static_assert(!RAW || MT == 1, "at most one row tile quantizes in the launch");
   static_assert(!SPLIT || (FMT != kSgBlock && !RAW), "quantized INT8 / FP8 rows split");
+  static_assert(!APART || (FMT != kSgBlock && !SPLIT), "block scales are slotted by wave");
   using L = SgLds<FMT, RAW, MT, NT, R, XH, SW>;
   using Acc = typename SgAcc<FMT>::T;
   constexpr bool BLOCK = FMT == kSgBlock;
@@ -260,8 +264,9 @@ __global__ void __launch_bounds__(64 * NW) stream_gemm_kernel(StreamArgs a) {
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
   const uint32_t lds0 = lds_base + wave * L::Wave;
 
-  // this wave's K blocks: kbeg + i * NW
-  int kbeg = wave, nblocks = KB;
+  // this wave's K blocks: kbeg + i * kstep
+  constexpr int kstep = APART ? 1 : NW;
+  int kbeg = APART ? wave * (KB / NW) : wave, nblocks = KB;
   if constexpr (SPLIT) {
     const int lo = (int)blockIdx.z * a.split_blocks;
     nblocks = min(KB - lo, a.split_blocks);
@@ -304,7 +309,7 @@ __global__ void __launch_bounds__(64 * NW) stream_gemm_kernel(StreamArgs a) {
   // K tails (K % 128 != 0): the last block's chunks past K are not fetched
   // (zeros), in the weights as in the activations
   auto issue_w = [&](int i, int q, bool none) {
-    const int kb = kbeg + i * NW;
+    const int kb = kbeg + i * kstep;
     const int32_t so = __builtin_amdgcn_readfirstlane(none ? 0 : kb * 128);
     const bool tail = !BLOCK && ktail != 128 && kb == KB - 1;
 #pragma unroll
@@ -350,7 +355,7 @@ __global__ void __launch_bounds__(64 * NW) stream_gemm_kernel(StreamArgs a) {
     if (lane < 16 * MT && row0 + lane < row_end) vxs = (a.gather ? gat[lane] : row0 + lane) * KB * 4;
   }
   auto issue_x = [&](int i, int q, bool none) {
-    const int kb = none ? 0 : kbeg + i * NW;
+    const int kb = none ? 0 : kbeg + i * kstep;
     const uint32_t b = lds0 + q * L::Stage + L::W;
     const int32_t so = __builtin_amdgcn_readfirstlane(kb * (RAW ? 256 : 128));
     const bool tail = !BLOCK && ktail != 128 && kb == KB - 1;
@@ -418,7 +423,7 @@ __global__ void __launch_bounds__(64 * NW) stream_gemm_kernel(StreamArgs a) {
       uint8_t* frag = mine + L::Frag;
       const uint16_t q2 = sg_quant2<FMT, DT>(*(const uint32_t*)(xf + lane * 4), row_s, row_rs, row_ok);
       // zeros past K whatever the scale: 0 / 0 under a given scale of zero is NaN
-      *(uint16_t*)(frag + lane * 2) = (kbeg + i * NW) * 128 + lane * 2 < K ? q2 : (uint16_t)0;
+      *(uint16_t*)(frag + lane * 2) = (kbeg + i * kstep) * 128 + lane * 2 < K ? q2 : (uint16_t)0;
       xf = frag;
     } else if constexpr (RAW) {
       uint8_t* frag = mine + L::Frag;
@@ -560,11 +565,23 @@ static inline SgForm sg_quantized_form(bool block, int64_t m, int64_t n, int K, 
   return sg_form(sg_tiles(n, sw), (int)((m + 15) / 16), block ? m <= 16 && K >= 2048 : m == 1 && K > 2048);
 }
 
-template <int FMT, bool RAW, int MT, int NT, int NW, int R, int XH, bool SW, int DT, bool SPLIT = false>
+// Whether the waves of a launch of at most 16 rows take K apart: with rows a
+// multiple of 4 KB long the 16 rows of a tile lie on the same memory channels
+// at one K, and NW waves at neighbouring K meet there; apart they do not.  INT8,
+// us, weights out of cache, together / apart: M = 2 N = 4096 K = 4096 9.1 / 8.7,
+// K = 8192 12.2 / 11.8, K = 16384 20.9 / 17.5, N = 8192 K = 16384 35.3 / 28.4, but
+// N = 1024 K = 8192 9.9 / 10.0 and N = 4096 K = 12288 15.0 / 15.1; M = 24
+// N = 4096 K = 16384 22.4 / 22.6.
+static inline bool sg_apart(int64_t n, int K, bool sw) {
+  return K % 4096 == 0 && sg_tiles(n, sw) >= tg_device_cus();
+}
+
+template <int FMT, bool RAW, int MT, int NT, int NW, int R, int XH, bool SW, int DT, bool SPLIT = false,
+          bool APART = false>
 static void sg_launch_form(const StreamArgs& a, int row_tiles, hipStream_t stream) {
   constexpr int cols = (SW ? 8 : 16) * NT;
   const dim3 grid((unsigned)((a.N + cols - 1) / cols), (unsigned)row_tiles, SPLIT ? (unsigned)a.splits : 1u);
-  hipLaunchKernelGGL((stream_gemm_kernel<FMT, RAW, MT, NT, NW, R, XH, SW, DT, SPLIT>), grid, dim3(64 * NW), 0, stream, a);
+  hipLaunchKernelGGL((stream_gemm_kernel<FMT, RAW, MT, NT, NW, R, XH, SW, DT, SPLIT, APART>), grid, dim3(64 * NW), 0, stream, a);
 }
 
 template <int FMT, bool RAW, int MT, int XH, bool SW, int DT>
@@ -579,6 +596,14 @@ static void sg_launch_rows(const StreamArgs& a, SgForm f, int row_tiles, hipStre
     if (a.splits > 1) {  // (narrow products: one tile a workgroup)
       if constexpr (MT == 2) sg_launch_form<FMT, RAW, MT, 1, 8, 2, XH, SW, DT, true>(a, row_tiles, stream);
       else sg_launch_form<FMT, RAW, MT, 1, 4, 3, XH, SW, DT, true>(a, row_tiles, stream);
+      return;
+    }
+  }
+  if constexpr (FMT != kSgBlock && MT == 1) {
+    if (sg_apart(a.N, a.K, SW)) {
+      if (f.nt == 1) sg_launch_form<FMT, RAW, MT, 1, 8, 2, XH, SW, DT, false, true>(a, row_tiles, stream);
+      else if (f.nw == 8) sg_launch_form<FMT, RAW, MT, 2, 8, 2, XH, SW, DT, false, true>(a, row_tiles, stream);
+      else sg_launch_form<FMT, RAW, MT, 2, 4, 2, XH, SW, DT, false, true>(a, row_tiles, stream);
       return;
     }
   }

@@ -63,6 +63,22 @@ def test_int8_rows_are_exact(cuda, n, k):
         assert np.array_equal(np32(out), want)
 
 
+# rows of a multiple of 4 KB against a tile per CU and more: the waves take K apart
+@pytest.mark.parametrize("n,k,tiles,waves", [(4104, 4096, 2, 8), (4096, 4096, 1, 8), (8200, 4096, 2, 4)])
+def test_int8_rows_of_aligned_pitch_are_exact(cuda, n, k, tiles, waves):
+    module = _fill(Int8Linear(k, n, True), _gen(n + k)).to(cuda)
+    for m in (1, 2, 16):
+        banner(f"stream int8 apart m={m} n={n} k={k}")
+        assert w8a8_route(m, n, k) == ("stream", tiles, waves, 1)
+        x = torch.randn(m, k, generator=_gen(m)).to(torch.bfloat16)
+        acc = torch.empty(m, n, dtype=torch.int32, device=cuda)
+        out = hip.int8_linear_forward(x.to(cuda), module, accumulators=acc)
+        want, _, _, want_acc = olinear.int8_forward(
+            np32(x), module.weight.cpu().numpy(), module.weight_scale.cpu().numpy(), np32(module.bias))
+        assert np.array_equal(acc.cpu().numpy().astype(np.int64), want_acc)
+        assert np.array_equal(np32(out), want)
+
+
 @pytest.mark.parametrize("n,k", SHAPES)
 def test_fp8_rows_match_oracle(cuda, n, k):
     module = _fill(Fp8Linear(k, n, True), _gen(n + k)).to(cuda)
