@@ -27,11 +27,12 @@ struct W4StreamArgs {
 struct W4StreamForm {
   int nt, ksplit;          // column tiles of a workgroup, K splits
 };
+// How the rows reach the launch: fp16 read where they are, bf16 read where they
+// are and converted in the loop, or gathered (as fp16) through a permutation.
+enum W4Rows { kW4RowsInPlace, kW4RowsConverted, kW4RowsGathered };
 // Whether the streaming GEMM is the faster one for these sizes (17 rows up),
-// and its form, with at most max_splits K splits.  fp16_in_place: x is fp16 and
-// is read where it is (no act-order gather before).
-bool w4_stream_form(int M, int N, int K, bool fp16_in_place, int swiglu, int cus, int max_splits,
-                    W4StreamForm* f);
+// and its form, with at most max_splits K splits.
+bool w4_stream_form(int M, int N, int K, W4Rows rows, int swiglu, int cus, int max_splits, W4StreamForm* f);
 void launch_w4_stream(const W4StreamArgs& a, const W4StreamForm& f, hipStream_t stream);
 
 }  // namespace kq

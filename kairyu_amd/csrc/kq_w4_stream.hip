@@ -239,16 +239,30 @@ w4a16_stream_kernel(W4StreamArgs a) {
 // fp16 but 43 against 36 in bf16, N = 4096 K = 14336 30.2 against 27.3).  Above
 // 32 rows the fp16 rows of a narrow, long-K layer still gain (19.8 against 23.8
 // us at N = 4096, K = 14336), but rows converted in the loop or gathered first
-// do not: bf16 K = 18944 28.1 against 26.3 us, K = 14336 23.3 / 23.9, gathered
-// 24.7 / 25.3; K = 4096 gains in every form (bf16 13.8 against 15.9).
+// do not past K = 8192 where K is split: bf16 N = 4096 K = 14336 23.3 / 23.9,
+// N = 3584 K = 18944 28.1 / 26.3, gathered N = 4096 K = 14336 24.7 / 25.3.  And
+// with K whole on less than two thirds of the CUs, where the tile kernel splits
+// it three ways, rows converted in the loop stop gaining at K = 4096 (N = 8448,
+// M = 33, K = 3072 17.4 / 17.7, 4096 21.0 / 19.9, 8192 36.0 / 28.8), gathered ones
+// at K = 6144 and 41 rows (M = 48, K = 4096 20.5 / 21.5, 6144 27.2 / 25.9; M = 33
+// 23.6 / 24.9).
 //
 // Columns: the NT with the least rounds of workgroups over the CUs times
 // columns, the wider one of two that tie (N = 28672: 8 26.0 us, 6 41, 4 37;
 // N = 37888: 10 31.1 us, 8 44.7; N = 57344 K = 8192: 8 82 us, 10 104).  CUs
 // left over take K splits, down to one stage per wave (N = 1024 K = 4096,
 // M = 32: 8 splits 7.9 us, 4 8.3; N = 4096 K = 4096: 4 splits 9.8 us, 2 11.1).
-bool w4_stream_form(int M, int N, int K, bool fp16_in_place, int swiglu, int cus, int max_splits,
-                    W4StreamForm* f) {
+//
+// SwiGLU here keeps K whole; where the plain product would split it, that with
+// the elementwise pass (about 3.5 us more) is the faster one as soon as the
+// split saves more than that.  A wave's stage of 128 k takes about 0.85 us of
+// fp16 rows up to 32 (0.72 where they were gathered just before), 1.2 above, and
+// 1.3 / 1.8 of rows converted in the loop:
+// fused against two passes, us, I = 1536 M = 17 / 33, fp16 K = 2048 9.6 / 12.4
+// and 10.2 / 11.6, K = 4096 13.0 / 17.1 and 11.9 / 13.7; bf16 K = 2048 11.4 / 15.3
+// and 10.8 / 12.4, K = 8192 27.1 / 36.7 and 16.1 / 19.4 (the tile kernel's two
+// passes 19.6 / 21.1); I = 3072 fp16 K = 4096 13.2 / 17.4 and 13.8 / 16.2.
+bool w4_stream_form(int M, int N, int K, W4Rows rows, int swiglu, int cus, int max_splits, W4StreamForm* f) {
   if (M > 48) return false;
   const int tiles = (N + 15) / 16, nst = K / 128;
   f->nt = 4;
@@ -261,8 +275,17 @@ bool w4_stream_form(int M, int N, int K, bool fp16_in_place, int swiglu, int cus
     }
   }
   const int blocks = (tiles + f->nt - 1) / f->nt;
-  f->ksplit = swiglu ? 1 : std::max(1, std::min({cus / blocks, max_splits, nst / kW4sWaves}));
-  return M <= 32 || fp16_in_place || f->ksplit == 1 || K <= 8192;
+  const int splits = std::max(1, std::min(cus / blocks, nst / kW4sWaves));
+  if (swiglu) {
+    f->ksplit = 1;
+    const float stage = rows == kW4RowsConverted ? (M > 32 ? 1.8f : 1.3f) : (M > 32 ? 1.2f : rows == kW4RowsGathered ? 0.72f : 0.85f);
+    return (nst - nst / splits) * stage < 3.5f * kW4sWaves;
+  }
+  f->ksplit = std::max(1, std::min(splits, max_splits));
+  if (M <= 32 || rows == kW4RowsInPlace) return true;
+  if (f->ksplit > 1) return K <= 8192;
+  const bool idle = 3 * ((N + 127) / 128) <= cus;
+  return !idle || (rows == kW4RowsConverted ? K < 4096 : M <= 40 || K < 6144);
 }
 
 template <int MT, bool BF16>

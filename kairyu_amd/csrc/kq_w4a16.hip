@@ -1728,10 +1728,10 @@ static void launch_gv(const W4Args& a, const GvPlan& p, int xdt, int S, int spg,
 // read in place (16-byte aligned) or gathered through the act-order permutation.
 static bool stream_form(const W4Args& a, int gmode, int max_splits, W4StreamForm* f) {
   const bool permuted = gmode == kGroupsPermuted;
+  const W4Rows rows = permuted ? kW4RowsGathered : a.x_dtype == KQ_DTYPE_F16 ? kW4RowsInPlace : kW4RowsConverted;
   return a.M > 16 && prefill_applies(a, gmode) && (int64_t)a.M * a.ldx < ((int64_t)1 << 30) &&
          (permuted || (((uintptr_t)a.x & 15) == 0 && a.ldx % 8 == 0)) &&
-         w4_stream_form(a.M, a.N, a.K, !permuted && a.x_dtype == KQ_DTYPE_F16, a.swiglu, device_cus(),
-                        max_splits, f);
+         w4_stream_form(a.M, a.N, a.K, rows, a.swiglu, device_cus(), max_splits, f);
 }
 
 static void run_w4_stream(const W4Args& a, const W4StreamForm& f, int gmode, uint16_t* x16, float* partials,
@@ -2107,7 +2107,9 @@ extern "C" int kq_w4a16_tiled_swiglu_gemm(const void* x, int x_dtype, const int3
   if (a.M > 0 && (gv_plan(a, kGptq, gmode, &gp, &s_, &spg_) || (a.M > 64 && prefill_applies(a, gmode))))
     return run_w4(what, kGptq, a, gmode, workspace, workspace_bytes, (hipStream_t)stream);
   // 17 to 48 rows: the streaming GEMM's SwiGLU epilogue (I = 14336, K = 4096,
-  // M = 48: 26.0 against 35.7 us for the tile GEMM and the elementwise pass).
+  // M = 48: 26.0 against 35.7 us for the tile GEMM and the elementwise pass),
+  // but where K splits save more than the elementwise pass costs
+  // (w4_stream_form).
   // The scratch that the two passes below ask for stays the call's condition.
   W4StreamForm sf{};
   if (stream_form(a, gmode, 1, &sf) && workspace != nullptr &&

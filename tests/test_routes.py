@@ -75,3 +75,26 @@ def test_few_rows_of_narrow_long_products_split_k(m, n, k, splits):
 def test_sixteen_waves_are_for_one_row(m, n, k, waves):
     assert w8a8_route(m, n, k).waves == waves
     assert w8a8_route(m, n, k, swiglu=True) == w8a8_route(m, n, k)
+
+
+@pytest.mark.parametrize("dtype,gathered,m,width,k,kernel", [
+    (torch.float16, False, 32, 14336, 4096, "stream"), (torch.bfloat16, True, 48, 11008, 4096, "stream"),
+    (torch.float16, False, 17, 2048, 2048, "stream"), (torch.bfloat16, False, 17, 2048, 2048, "tile"),
+    (torch.bfloat16, False, 48, 3072, 1024, "stream"), (torch.float16, False, 48, 2752, 4096, "tile"),
+    (torch.bfloat16, False, 17, 3456, 5120, "tile"), (torch.bfloat16, True, 33, 3584, 8192, "tile")])
+def test_w4_swiglu_keeps_k_whole_only_where_that_is_short(dtype, gathered, m, width, k, kernel):
+    """Else two passes, whose plain product streams with its K split ("tile":
+    not this kernel's fused form)."""
+    assert w4a16_route(dtype, gathered, m, 2 * width, k, 128, swiglu=True).kernel == kernel
+    if kernel == "tile":
+        plain = w4a16_route(dtype, gathered, m, 2 * width, k, 128)
+        assert plain.kernel == "stream" and plain.splits > 1
+
+
+@pytest.mark.parametrize("dtype,gathered,m,n,k,kernel", [
+    (torch.bfloat16, False, 33, 10240, 8192, "tile"), (torch.bfloat16, False, 32, 10240, 8192, "stream"),
+    (torch.float16, False, 48, 10240, 8192, "stream"), (torch.bfloat16, True, 48, 10240, 8192, "tile"),
+    (torch.bfloat16, True, 40, 10240, 8192, "stream"), (torch.bfloat16, False, 48, 9472, 3584, "stream"),
+    (torch.bfloat16, False, 48, 11008, 8192, "stream")])
+def test_w4_rows_leave_the_cus_idle_on_short_k_only(dtype, gathered, m, n, k, kernel):
+    assert w4a16_route(dtype, gathered, m, n, k, 128).kernel == kernel
