@@ -1,8 +1,7 @@
 """Benchmark of the quantized-linear hot path on one MI355X.
 
-Headline (``value``): GPTQ act-order W4A16 (N=28672,
-K=4096, group 128) at decode size M=16, as whole-op HBM throughput in GB/s of
-algorithmic bytes.  One step = one forward of the quantized linear on one
+Headline (``value``): GPTQ act-order W4A16 (N=28672, K=4096, group 128) at
+decode size M=16, as whole-op HBM throughput in GB/s of algorithmic bytes.  One step = one forward of the quantized linear on one
 batch; weights rotate over enough distinct HBM copies (> 256 MB MALL) that no
 step is served from the Infinity Cache.  `--steps` steps are captured in one
 HIP graph; each timing sample replays it back to back for at least 200 steps
@@ -31,7 +30,9 @@ Qwen2-7B for AWQ, GPTQ act-order and FP8, each row with
     workload on this host's cores, and the device output on the same sample
     judged against the oracle with the test suite's criteria
     (``oracle.parity``).
-``context`` holds the reference microbenchmark's own setup (N = K = 4096, M
+The printed line holds a few numbers of each row, so that it stays a few KB;
+``--rows FILE`` writes them whole.  ``context`` holds the reference
+microbenchmark's own setup (N = K = 4096, M
 in {1, 128}, bf16, seed 205, four formats) timed its way and this bench's
 way, next to its published numbers on its own GPU (``--no-context`` skips).
 The top-level ``cpu_baseline`` is the headline row's.  ``peaks`` holds the
@@ -724,6 +725,8 @@ def main() -> int:
                         help="only measure the box's streaming-read and MFMA-loop ceilings")
     parser.add_argument("--no-peaks", action="store_true",
                         help="skip the measured ceilings in a full run")
+    parser.add_argument("--rows", default=None, metavar="FILE",
+                        help="write every sweep and context row whole, as JSON")
     parser.add_argument("--no-context", action="store_true",
                         help="skip the reference microbenchmark's context rows")
     args = parser.parse_args()
@@ -842,7 +845,7 @@ def main() -> int:
         "dtype": "fp16",
         "data": "synthetic (seeded torch.Generator; no checkpoint)",
         "config": {
-            "workload": "BASELINE configs[1]: GPTQ act-order W4A16 N=28672 K=4096 group=128, M=16 decode",
+            "workload": "GPTQ act-order W4A16 N=28672 K=4096 group=128, M=16 decode",
             "m": 16, "n": 28672, "k": 4096, "group_size": 128, "act_order": True,
             "x_dtype": "float16", "weight_copies": head["copies"],
         },
@@ -866,8 +869,22 @@ def main() -> int:
         "sweep": sweep,
         "context": context,
     }
-    print(json.dumps(line), flush=True)
+    if args.rows:
+        Path(args.rows).write_text(json.dumps({"sweep": sweep, "context": context}) + "\n")
+    # the line holds a few numbers of each row (--rows writes them whole)
+    line["sweep"] = {"columns": ["workload", "us", "gb_per_s", "tflops", "gemm_us", "gemm_frac", "parity"],
+                     "rows": [_short(row) for row in sweep]}
+    line["context"] = {"columns": ["scheme", "m", "eager_us", "graph_us", "reference_rtx_pro_6000_us"],
+                       "rows": [[c["scheme"], c["shape"]["m"], c["eager_median_us"], c["graph_us"],
+                                 c["reference_rtx_pro_6000_us"]] for c in context or ()]}
+    print(json.dumps(line, separators=(",", ":")), flush=True)
     return 0
+
+
+def _short(row: dict) -> list:
+    gemm = row.get("gemm") or {}
+    return [row["workload"], row["us"], row["gb_per_s"], row["tflops"], gemm.get("us"), gemm.get("frac"),
+            (row.get("parity") or {}).get("verdict")]
 
 
 if __name__ == "__main__":
