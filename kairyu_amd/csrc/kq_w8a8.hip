@@ -243,8 +243,8 @@ static void reduce_splits(const void* partials, int splits, const Epi& ep, hipSt
 // 17.1 / 13.0 / 13.4, 26.4 / 16.6 / 15.6; N = 1536 (whole / 2) M = 17 K = 8192
 // 12.3 / 12.7, K = 12288 15.7 / 14.7.
 static int stream_splits(int64_t m, int64_t n, int64_t k) {
-  const int64_t room = tg_device_cus() / ((n + 15) / 16), kb = (k + 127) / 128;
   if (m <= 16) return 1;
+  const int64_t room = tg_device_cus() / ((n + 15) / 16), kb = (k + 127) / 128;
   if (room >= 8 && kb >= (m > 32 ? 96 : 128)) return 8;
   if (room >= 4 && kb >= (m > 48 ? 32 : m > 32 ? 40 : 64)) return 4;
   return room >= 2 && kb >= 96 ? 2 : 1;
