@@ -105,8 +105,8 @@ int kq_w8a8_fp8_gemm(const uint8_t* xq, const float* xscale, const uint8_t* w,
  * [m, k] (row pitch ldx) is quantized exactly as kq_act_quant_i8 /
  * kq_act_quant_fp8 would (INT8 dynamic; FP8 scale_mode 0 dynamic, 1 static
  * scale_in[0], 2 per-row scale_in[m]) and multiplied with w as
- * kq_w8a8_i8_gemm / kq_w8a8_fp8_gemm do.  Small decode batches quantize
- * inside the GEMM launch; other shapes stage the quantized rows in the
+ * kq_w8a8_i8_gemm / kq_w8a8_fp8_gemm do.  One row is quantized inside the GEMM
+ * launch; other shapes stage the quantized rows in the
  * workspace (kq_w8a8_linear_workspace_size bytes).  Replaces the
  * _quantize_activation + GEMM pair of int8_linear_forward / fp8_linear_forward
  * (quant_gemm_gpu.py:538-572, :596-687). */
@@ -128,10 +128,10 @@ size_t kq_w8a8_linear_workspace_size(int64_t m, int64_t n, int64_t k);
  * rows), and out [m][i_width] (activation dtype) = silu(g) * u for gate
  * column c and up column i_width + c, with the roundings of
  * kq_w8a8_*_linear followed by kq_swiglu (bit-identical to that pair).
- * Prefill shapes apply SwiGLU in the tile engine's epilogue and shapes of
- * m <= 64 in the weight-streaming GEMM's:
- * the [m][2I] projection never reaches memory; other shapes run the pair
- * through the workspace.  Replaces the reference MLP's act_fn(gate(x)) *
+ * SwiGLU is applied in the epilogue of the weight-streaming GEMM (m <= 64), of
+ * the panel GEMM (m <= 256) and of the tile engine, or in the reduce where one
+ * of the first two splits K: the [m][2I] projection never reaches memory.  Other
+ * shapes run the pair through the workspace.  Replaces the reference MLP's act_fn(gate(x)) *
  * up(x) (kairyu/models/layers.py:243-244) over its packed projections
  * (kairyu/models/packed_linear.py:58-149) for FP8 / INT8 W8A8. */
 int kq_w8a8_i8_swiglu_linear(const void* x, int x_dtype, int64_t ldx, const int8_t* w,
@@ -336,7 +336,7 @@ int kq_block_fp8_gemm(const uint8_t* xq, const float* xs, const uint8_t* w, cons
                       int64_t n, int64_t k, void* stream);
 
 /* kq_act_quant_fp8_blocks of x (fp16/bf16 [m, k], row pitch ldx) and
- * kq_block_fp8_gemm in one call, out [m, n] in x_dtype: decode batches are
+ * kq_block_fp8_gemm in one call, out [m, n] in x_dtype: up to 16 rows are
  * quantized inside the GEMM launch, other shapes through the workspace
  * (kq_block_fp8_workspace_size bytes).  Replaces finegrained_fp8_linear
  * (deepseek_v4_moe_gpu.py:60-74) for BlockFp8Linear. */
@@ -348,7 +348,9 @@ size_t kq_block_fp8_workspace_size(int64_t m, int64_t k);
 /* out [m, i_width] = silu(gate) * up of two block-FP8 projections [i_width, k]
  * of the same x, m <= 128, with the roundings of the two linears followed by
  * torch's silu and product (each projection's bias may be null, both of
- * bias_dtype).  Replaces act_fn(gate(x)) * up(x) of the expert MLP
+ * bias_dtype).  Past 64 rows the bits are those of that pair; up to 64 the fp32
+ * K blocks of a column may be added in another order than a narrower linear adds
+ * them, each sum within the same bound.  Replaces act_fn(gate(x)) * up(x) of the expert MLP
  * (kairyu/models/moe.py:27-83). */
 int kq_block_fp8_swiglu_linear(const void* x, int x_dtype, int64_t ldx, const uint8_t* w_gate,
                                const float* s_gate, const uint8_t* w_up, const float* s_up,

@@ -231,8 +231,9 @@ def device_supported(index: int) -> bool:
 
 
 class WorkspacePool:
-    """Per-device scratch buffers (split-K partials, act-order activation
-    gather, MoE intermediates), one per device, reused by every call.
+    """Per-device scratch buffers (W8A8 quantized rows, split-K partials,
+    act-order activation gather, MoE intermediates), one per device, reused by
+    every call but the block-FP8 linears', which take scratch of their own.
 
     Growth is geometric: a call needing more than the current buffer gets
     ``max(need, 2 * current)`` bytes, so a sequence of ever larger calls

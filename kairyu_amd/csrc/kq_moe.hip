@@ -188,7 +188,14 @@ static inline int moe_nrb(int64_t routed_rows, int64_t experts) {
 // (a further tile reads the expert's weights again).  C5's widths, whole call
 // (graph replay; before, after): 16 tokens (8-row tiles) 116 -> 78 us, 32
 // (8) 157 -> 97, 64 (16) 159 -> 117, 128 (32) 161 -> 134, 256 (32) 165 ->
-// 143; 512 tokens take 174 us with 256-row tiles and 250 with 64-row ones.
+// 143; 512 tokens take 174 us with 256-row tiles and 250 with 64-row ones.  Other
+// widths (weights out of cache, the line's upper ends): H = 2048 I = 1024, 64
+// experts top 8 117 -> 102; 4096 / 1536, 32 top 8 188 -> 134; 1024 / 512, 32 top 4
+// at 16 tokens 52 -> 40.  The host does not see the routing, so the lines are those
+// of even and Zipf-like ones (C5, 256 tokens: 167 -> 140, 170 -> 135); an expert
+// of many rows reads its weights once per row tile, and such a routing can lose:
+// all 256 tokens in 16 of the 128 experts 74 -> 89, 192 71 -> 78, 128 69 -> 64, all
+// 256 in the same 8 77 -> 79.
 static inline int moe_stream_rows(int64_t routed_rows, int64_t experts) {
   if (routed_rows <= 2 * experts) return 8;
   if (routed_rows <= 6 * experts) return 16;

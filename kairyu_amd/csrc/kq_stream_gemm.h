@@ -537,9 +537,9 @@ __global__ void __launch_bounds__(64 * NW) stream_gemm_kernel(StreamArgs a) {
 // memory.  (FP8, us, 16 waves against 8: one row N = 1024 K = 4096 4.6 / 4.8, K =
 // 8192 6.4 / 6.8, but N = 256 K = 2048 3.5 / 3.3, a K block a wave; with more
 // rows the waves' sums cost what their loads gain: N = 512 M = 8 K = 4096 6.8 /
-// 6.7, K = 16384 13.7 / 13.1.)  Block FP8 takes 16 waves up to its first 16 rows'
-// form, whose waves quantize, from a K block a wave.  Up to one tile per CU, one
-// tile and 8 waves, so that every CU streams; up to two, two tiles (one round of
+// 6.7, K = 16384 13.7 / 13.1.)  Block FP8 takes them from a K block a wave, up to
+// 16 rows (8 where the launch quantizes).  Up to one tile per CU, one tile and 8
+// waves, so that every CU streams; up to two, two tiles (one round of
 // workgroups); beyond, two tiles and 4 waves, several workgroups per CU, so
 // that one's prologue and epilogue run under another's stream.  Measured, FP8
 // (us; graph replay, weights rotating past the MALL): N = K = 4096 M = 8 5.6,

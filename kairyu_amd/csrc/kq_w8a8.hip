@@ -9,14 +9,19 @@
 //         (kairyu/quant/fp8.py:48-56, linear.py:463-469).
 //
 // Kernels:
-//   * M <= 64: the weight-streaming kernel of kq_stream_gemm.h.  HBM-bound.
-//   * M <= 256: the panel kernel of kq_panel_gemm.h where its panels fill the
-//     CUs (and 33 to 64 rows against many weight rows).
-//   * M > 64 with at least one 256x256 tile per CU: the persistent tile
-//     engine of kq_tile_gemm.h (LDS DMA double buffering, XCD-grouped tiles).
-//   * other M > 64: 128x128x128 workgroup tiles, 4 waves of 64x64, LDS
+//   * M <= 64: the weight-streaming kernel of kq_stream_gemm.h, HBM-bound;
+//     narrow products of 17 rows up split K over workgroups (stream_splits).
+//   * M <= 256: the panel kernel of kq_panel_gemm.h (and 33 to 64 rows against
+//     many weight rows), K split over workgroups where its panels leave half the
+//     CUs idle (pg_form).
+//   * other M > 64 with one 256x256 tile per CU, or half as many units with K
+//     split: the persistent tile engine of kq_tile_gemm.h (LDS DMA double
+//     buffering, XCD-grouped tiles).
+//   * the rest: 128x128x128 workgroup tiles, 4 waves of 64x64, LDS
 //     double buffer with an XOR chunk swizzle (twice the workgroups of the
 //     256x256 engine for shapes that would leave CUs idle).
+// The raw accumulators of every K split are added in split order by one reduce
+// launch with the epilogue (kq_splitk.h).
 #include "kq_common.h"
 #include "kq_panel_gemm.h"
 #include "kq_splitk.h"
@@ -550,7 +555,8 @@ extern "C" int kq_w8a8_fp8_linear(const void* x, int x_dtype, int64_t ldx, const
 // gate columns [n0, n0 + 128) with up columns [I + n0, I + n0 + 128), so the
 // [M, 2I] projection output never reaches memory.  Shapes of M <= 64 run the
 // weight-streaming kernel, up to 256 rows the panel kernel, with the SwiGLU
-// epilogue (each 16-row weight tile is 8 gate rows and the matching 8 up rows).  Other shapes run the packed
+// epilogue (each 16-row weight tile is 8 gate rows and the matching 8 up rows),
+// which a split K puts off to the reduce.  Other shapes run the packed
 // linear into the workspace and the elementwise pass.  All produce the bits
 // of the packed linear followed by kq_swiglu.
 static bool swiglu_fused_applies(int64_t m, int64_t i_width, int64_t k, const void* x, int64_t ldx,

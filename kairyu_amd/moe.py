@@ -143,7 +143,9 @@ class BlockFp8ExpertMlp(nn.Module):
     def _fused_swiglu(self, hidden: torch.Tensor) -> bool:
         """Whether gate, up and their SwiGLU run as one launch: a batch of few
         rows through two plain block-FP8 projections (no hooks of their own or of
-        every module, no other forward bound) of equal widths and alike biases."""
+        every module, no other forward bound) of equal widths and alike biases.
+        The outputs are those of the two linears up to the order in which the
+        fp32 sums of K blocks are added (up to 64 rows)."""
 
         from kairyu_amd.kernels import quant_gemm_hip as hip
 
